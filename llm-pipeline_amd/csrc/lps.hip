@@ -399,6 +399,37 @@ hipError_t launch_softmax_reg(const SoftmaxParams& S, const SmPlan& p, hipStream
   return hipGetLastError();
 }
 
+template <int DT, int ODT, typename T, bool NTL>
+hipError_t launch_lmhead(LmHeadParams P, hipStream_t s) {
+  P.mtiles = (P.M + T::BM - 1) / T::BM;
+  P.tiles = P.mtiles * ((P.V + T::BN - 1) / T::BN);
+  hipLaunchKernelGGL((lmhead_kernel<DT, ODT, T, NTL>), dim3((unsigned)(P.tiles + 7) / 8 * 8), dim3(T::NT), 0, s, P);
+  return hipGetLastError();
+}
+// The tile shape by row count (figures in lps_lmhead.h): one row tile as long
+// as the weight's pass over HBM is the bound, so that it is read once and
+// streamed past the caches; 129 to 256 rows fill one 256-row tile (160 rows:
+// 363 us, two 128-row tiles 399); up to 384 rows three 128-row tiles beat two
+// of 256 (554 against 619 us), at 512 and 640 rows they do not (759 against
+// 627, 918 against 883).
+template <int DT, int ODT>
+hipError_t launch_lmhead_rows(const LmHeadParams& P, hipStream_t s) {
+  if (P.M <= 32) return launch_lmhead<DT, ODT, LmTile<32, 128, 1, 4, 128, 3, 1>, true>(P, s);
+  if (P.M <= 64) return launch_lmhead<DT, ODT, LmTile<64, 128, 1, 4, 128, 3, 1>, true>(P, s);
+  if (P.M <= 96) return launch_lmhead<DT, ODT, LmTile<96, 128, 1, 4, 64, 5, 1>, true>(P, s);
+  if (P.M <= 128) return launch_lmhead<DT, ODT, LmTile<128, 128, 4, 2, 64, 4, 2>, true>(P, s);
+  if (P.M > 256 && P.M <= 384) return launch_lmhead<DT, ODT, LmTile<128, 256, 2, 2, 64, 2, 1>, false>(P, s);
+  return launch_lmhead<DT, ODT, LmTile<256, 256, 4, 2, 64, 2, 2>, false>(P, s);
+}
+template <int DT>
+hipError_t dispatch_lmhead(const LmHeadParams& P, int out_dtype, hipStream_t s) {
+  switch (out_dtype) {
+    case LPS_DTYPE_F32: return launch_lmhead_rows<DT, LPS_DTYPE_F32>(P, s);
+    case LPS_DTYPE_BF16: return launch_lmhead_rows<DT, LPS_DTYPE_BF16>(P, s);
+    default: return launch_lmhead_rows<DT, LPS_DTYPE_F16>(P, s);
+  }
+}
+
 // Monotonicity of the hardware exp2 (v_exp_f32) over every non-NaN input:
 // thread t checks keys [k0 + 1024 t - 1, k0 + 1024 t + 1024) in float-key
 // order (each step against the one before it), counting the steps where the
@@ -748,7 +779,7 @@ int lps_lm_head(const lps_lm_head_args* a, void* stream) {
   if (reinterpret_cast<uintptr_t>(a->x) % 16 || reinterpret_cast<uintptr_t>(a->w) % 16 || a->x_stride % 8 ||
       a->w_stride % 8)
     return LPS_EINVAL;
-  if ((a->rows + LMH_BM - 1) / LMH_BM > 65535) return LPS_EINVAL;   // grid y
+  if (a->rows > LMH_MAX_ROWS) return LPS_EINVAL;
   LmHeadParams P{};
   P.x = a->x;
   P.w = a->w;
@@ -762,19 +793,9 @@ int lps_lm_head(const lps_lm_head_args* a, void* stream) {
   P.out_stride = a->rows > 1 ? a->out_stride : a->vocab;
   P.G = (a->vocab + LMH_BN - 1) / LMH_BN;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)P.G, (unsigned)((a->rows + LMH_BM - 1) / LMH_BM));
-#define LMH_LAUNCH(DT, ODT) hipLaunchKernelGGL((lmhead_kernel<DT, ODT, LMH_KC, LMH_NB>), grid, dim3(256), 0, s, P)
-  if (a->dtype == LPS_DTYPE_BF16) {
-    if (a->out_dtype == LPS_DTYPE_BF16) LMH_LAUNCH(LPS_DTYPE_BF16, LPS_DTYPE_BF16);
-    else if (a->out_dtype == LPS_DTYPE_F16) LMH_LAUNCH(LPS_DTYPE_BF16, LPS_DTYPE_F16);
-    else LMH_LAUNCH(LPS_DTYPE_BF16, LPS_DTYPE_F32);
-  } else {
-    if (a->out_dtype == LPS_DTYPE_BF16) LMH_LAUNCH(LPS_DTYPE_F16, LPS_DTYPE_BF16);
-    else if (a->out_dtype == LPS_DTYPE_F16) LMH_LAUNCH(LPS_DTYPE_F16, LPS_DTYPE_F16);
-    else LMH_LAUNCH(LPS_DTYPE_F16, LPS_DTYPE_F32);
-  }
-#undef LMH_LAUNCH
-  return hipGetLastError() == hipSuccess ? LPS_OK : LPS_ELAUNCH;
+  const hipError_t e = a->dtype == LPS_DTYPE_BF16 ? dispatch_lmhead<LPS_DTYPE_BF16>(P, a->out_dtype, s)
+                                                  : dispatch_lmhead<LPS_DTYPE_F16>(P, a->out_dtype, s);
+  return e == hipSuccess ? LPS_OK : LPS_ELAUNCH;
 }
 
 int lps_softmax(const lps_softmax_args* a, void* stream) {

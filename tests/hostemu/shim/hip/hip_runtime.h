@@ -319,6 +319,7 @@ template <typename T> inline T atomicCAS(T* p, T cmp, T v) {
 #define __builtin_amdgcn_fence(order, scope) __atomic_thread_fence(order)
 #define __builtin_amdgcn_s_waitcnt(n) ((void)0)
 #define __builtin_amdgcn_s_sleep(n) std::this_thread::yield()
+#define __builtin_amdgcn_s_setprio(n) ((void)0)
 #define __builtin_amdgcn_s_memrealtime() ((uint64_t)0)
 // HW_REG_XCC_ID: the XCD a block id is dispatched to (round-robin over 8)
 #define __builtin_amdgcn_s_getreg(reg) ((int)(::lps_emu::t_block.x & 7u))
@@ -396,12 +397,30 @@ inline T __shfl(T v, int src, int w = 64) {
   return lps_emu::xchg<T>(v, [&](const uint64_t* b, uint64_t) { return lps_emu::from_bits<T>(b[src & 63]); });
 }
 
-// Matrix-core instructions are not emulated (the LM-head kernel is not run here).
+// v_mfma_f32_32x32x16_{bf16,f16}: lane l holds A row and B column l % 32 at k =
+// 8 (l / 32) .. +7, and element i of the result is row 8 (i / 4) + 4 (l / 32) +
+// i % 4, column l % 32.
 template <typename A, typename C>
-inline C lps_emu_no_mfma(A, A, C c) {
-  fprintf(stderr, "hostemu: matrix-core instructions are not emulated\n");
-  abort();
+inline C lps_emu_mfma(A a, A b, C c) {
+  struct Ops { A v[2][64]; };
+  Ops o;
+  for (int m = 0; m < 2; m++) {
+    uint64_t h[2];
+    memcpy(h, m == 0 ? &a : &b, 16);
+    for (int p = 0; p < 2; p++)
+      lps_emu::xchg<uint64_t>(h[p], [&](const uint64_t* w, uint64_t) {
+        for (int l = 0; l < 64; l++) memcpy(reinterpret_cast<char*>(&o.v[m][l]) + 8 * p, &w[l], 8);
+        return (uint64_t)0;
+      });
+  }
+  const int l = lps_emu::lane();
+  for (int i = 0; i < 16; i++) {
+    const int row = 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), col = l & 31;
+    float s = c[i];
+    for (int k = 0; k < 16; k++) s += (float)o.v[0][row + 32 * (k >> 3)][k & 7] * (float)o.v[1][col + 32 * (k >> 3)][k & 7];
+    c[i] = s;
+  }
   return c;
 }
-#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) lps_emu_no_mfma((a), (b), (c))
-#define __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, x, y, z) lps_emu_no_mfma((a), (b), (c))
+#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) lps_emu_mfma((a), (b), (c))
+#define __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, x, y, z) lps_emu_mfma((a), (b), (c))

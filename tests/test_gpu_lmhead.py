@@ -93,3 +93,22 @@ def test_softmax_from_stats_equals_softmax(dev):
     torch.testing.assert_close(p.double().cpu(), ref, atol=1e-7, rtol=2 ** -8)
     p2, lse = fused_softmax(logits, row_stats=stats, return_lse=True)
     torch.testing.assert_close(lse.double().cpu(), torch.logsumexp(logits.double().cpu(), dim=-1), atol=2e-5, rtol=1e-6)
+
+
+@pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 96, 97, 128, 129, 256, 257, 384, 385])
+@pytest.mark.parametrize("V,H,dtype,out_dtype", [(301, 1040, torch.bfloat16, None),            # odd rows, a part of a stage
+                                                 (640, 1024, torch.float16, torch.float32),    # whole stages
+                                                 (260, 208, torch.float16, torch.bfloat16),    # fewer stages than buffers
+                                                 (129, 16, torch.bfloat16, torch.float16)])    # no whole stage
+def test_lm_head_tile_edges(dev, M, V, H, dtype, out_dtype):
+    """The row counts at which the tile shape changes, columns and hidden sizes
+    that end inside a tile or a stage; _check_logits' bound (one rounding of the
+    output type, fp32 accumulation).  The sums refer to the fp32 product max * log2 e,
+    whose rounding moves them by up to |max| * log2 e * 2^-24 * ln 2: logits of
+    deviation 2 (at most ~10) keep that under 1e-6, half of _check_stats' 2e-6."""
+    g = torch.Generator().manual_seed(M * 11 + V + H)
+    x = torch.randn((M, H), generator=g).to(dtype)
+    w = (torch.randn((V, H), generator=g) * (2.0 / H ** 0.5)).to(dtype)
+    out, stats = lm_head(x.to(dev), w.to(dev), out_dtype=out_dtype, return_stats=True)
+    _check_logits(out, _ref(x, w), H, 1.0)
+    _check_stats(out, stats)
