@@ -207,7 +207,6 @@ hipError_t launch_rg(rg::RgParams F, int flags, hipStream_t s) {
   // 1024-thread workgroup per row (the others return at once)
   KParams G = F.k;
   G.only_status = F.status;
-  G.plans = nullptr;
   return launch_gen<DT, VPE == 1 ? 1 : (DT == LPS_DTYPE_F32 ? 4 : 8)>(G, s);
 }
 
@@ -251,7 +250,6 @@ KParams row_block(const KParams& P, int r0, int nr, int es) {
   B.kept_ties = P.kept_ties ? P.kept_ties + r0 : nullptr;
   B.kept_count = P.kept_count ? P.kept_count + r0 : nullptr;
   B.row_path = P.row_path ? P.row_path + r0 : nullptr;
-  B.plans = P.plans ? P.plans + r0 : nullptr;
   B.allowed = P.allowed ? P.allowed + (int64_t)r0 * P.allowed_stride : nullptr;
   return B;
 }
@@ -326,8 +324,14 @@ struct SpecWs {
   int64_t* draws_d;   // [B*k]
   float* p_t;         // [B*(k+1)], then q_d
   float* q_d;         // [B*k]
-  int32_t* first_rej; // [B]
-  RowPlan* plans;     // [B*(k+1) + B*k]
+  // the residual option: each row's kept set and status (target rows, then
+  // draft rows), the chunks' records
+  float* cut;
+  int32_t* ties;
+  int32_t* status;
+  ResRec* rec;        // [B, chunks, 2]
+  uint64_t* rsum;     // [B, chunks]
+  uint32_t* count;    // [B]
   size_t bytes;
 };
 
@@ -342,8 +346,13 @@ SpecWs spec_layout(void* base, int B, int k, int V) {
   w.draws_d = ws_at<int64_t>(base, off + Rt * 8); off = align256(off + (Rt + Rd) * 8);
   w.p_t = ws_at<float>(base, off);
   w.q_d = ws_at<float>(base, off + Rt * 4); off = align256(off + (Rt + Rd) * 4);
-  w.first_rej = ws_at<int32_t>(base, off); off = align256(off + (size_t)B * 4);
-  w.plans = ws_at<RowPlan>(base, off); off = align256(off + (Rt + Rd) * sizeof(RowPlan));
+  w.cut = ws_at<float>(base, off); off = align256(off + (Rt + Rd) * 4);
+  w.ties = ws_at<int32_t>(base, off); off = align256(off + (Rt + Rd) * 4);
+  w.status = ws_at<int32_t>(base, off); off = align256(off + (Rt + Rd) * 4);
+  const size_t chunks = (size_t)B * (size_t)res_chunks(V);
+  w.rec = ws_at<ResRec>(base, off); off = align256(off + chunks * 2 * sizeof(ResRec));
+  w.rsum = ws_at<uint64_t>(base, off); off = align256(off + chunks * 8);
+  w.count = ws_at<uint32_t>(base, off); off = align256(off + (size_t)B * 4);
   w.bytes = off;
   return w;
 }
@@ -555,7 +564,6 @@ int sample_impl(const lps_sample_args* a, void* ws, size_t ws_bytes, void* strea
   P.kept_cut = a->kept_cut;
   P.kept_ties = a->kept_ties;
   P.kept_count = a->kept_count;
-  P.plans = nullptr;
   P.only_status = nullptr;
   P.row_path = a->row_path;
   P.allowed = a->allowed;
@@ -672,17 +680,21 @@ int lps_spec_verify(const lps_spec_args* a, void* stream) {
   P.query_prob = w.p_t;
   P.tokens = w.draws_t;
   P.row_status = a->row_status;
-  P.plans = w.plans;
-  // The Leviathan residual reads the general kernel's per-row plans; otherwise
-  // both row sets take the fast kernels (rows they cannot finish exactly go
-  // to the general kernel after them), with the same results.
+  if (lev) {
+    // the residual stage reads every row's kept set and status
+    P.kept_cut = w.cut;
+    P.kept_ties = w.ties;
+    if (!P.row_status) P.row_status = w.status;
+  }
+  // Both row sets take the fast kernels (rows they cannot finish exactly go to
+  // the general kernel after them).
   // Every row shares the temperature and top-p: the row-kind hint that skips
   // the kernel no row needs (T > 0: nucleus or pure rows; else greedy).
   const int hint = a->temperature > 0.0f ? LPS_FLAG_ROWS_NUCLEUS : LPS_FLAG_ROWS_TOPK;
   const int Rt = B * (k + 1), Rd = B * k;
-  bool vec = vec_ok(a->target_logits, a->dtype, V, k + 1, a->target_stride_b, a->target_stride_k);
+  const bool vec = vec_ok(a->target_logits, a->dtype, V, k + 1, a->target_stride_b, a->target_stride_k);
   const bool vec_d = vec_ok(a->draft_logits, a->dtype, V, k, a->draft_stride_b, a->draft_stride_k);
-  if (!lev && Rt + Rd <= RG_MAX_ROWS) {
+  if (Rt + Rd <= RG_MAX_ROWS) {
     // both row sets in one launch: the target rows, then the draft rows as
     // the second row segment (their own logits and layout, draws skipped);
     // the outputs of the two sets are contiguous in the workspace
@@ -696,42 +708,58 @@ int lps_spec_verify(const lps_spec_args* a, void* stream) {
     J.skip_draw2 = 1;
     if (run_sample(J, a->dtype, vec && vec_d, w.fast, w.fast_bytes, hint, s) != hipSuccess) return LPS_ELAUNCH;
   } else {
-  if ((lev ? dispatch_gen(a->dtype, vec, P, s) : run_sample(P, a->dtype, vec, w.fast, w.fast_bytes, hint, s)) !=
-      hipSuccess)
-    return LPS_ELAUNCH;
+    if (run_sample(P, a->dtype, vec, w.fast, w.fast_bytes, hint, s) != hipSuccess) return LPS_ELAUNCH;
 
-  // draft rows: probability of each draft token only
-  KParams D = P;
-  D.logits = a->draft_logits;
-  D.R = B * k;
-  D.rows_inner = k;
-  D.stride_outer = a->draft_stride_b;
-  D.stride_inner = a->draft_stride_k;
-  D.uniforms = nullptr;
-  D.query_inner = k;
-  D.query_prob = w.q_d;
-  D.tokens = w.draws_d;
-  D.row_status = a->row_status ? a->row_status + (size_t)B * (k + 1) : nullptr;
-  D.skip_draw = 1;
-  D.plans = w.plans + (size_t)B * (k + 1);
-  // (planned for both row sets' count, for which the workspace is sized)
-  if ((lev ? dispatch_gen(a->dtype, vec_d, D, s) : run_sample(D, a->dtype, vec_d, w.fast, w.fast_bytes, hint, s, Rt + Rd)) !=
-      hipSuccess)
-    return LPS_ELAUNCH;
+    // draft rows: probability of each draft token only
+    KParams D = P;
+    D.logits = a->draft_logits;
+    D.R = Rd;
+    D.rows_inner = k;
+    D.stride_outer = a->draft_stride_b;
+    D.stride_inner = a->draft_stride_k;
+    D.uniforms = nullptr;
+    D.query_inner = k;
+    D.query_prob = w.q_d;
+    D.tokens = w.draws_d;
+    D.row_status = P.row_status ? P.row_status + Rt : nullptr;
+    D.kept_cut = P.kept_cut ? P.kept_cut + Rt : nullptr;
+    D.kept_ties = P.kept_ties ? P.kept_ties + Rt : nullptr;
+    D.skip_draw = 1;
+    // (planned for both row sets' count, for which the workspace is sized)
+    if (run_sample(D, a->dtype, vec_d, w.fast, w.fast_bytes, hint, s, Rt + Rd) != hipSuccess) return LPS_ELAUNCH;
   }
 
-  hipLaunchKernelGGL(spec_epilogue_kernel, dim3((B + 255) / 256), dim3(256), 0, s, B, k, a->temperature, w.p_t,
-                     w.q_d, w.draws_t, a->draft_tokens, a->u_accept, a->n_accepted, a->tokens, a->accept,
-                     a->p_target, a->q_draft, lev ? 1 : 0, w.first_rej);
-  if (hipGetLastError() != hipSuccess) return LPS_ELAUNCH;
-  if (lev) {
-    const bool vt = vec_ok(a->target_logits, a->dtype, V, k + 1, a->target_stride_b, a->target_stride_k) &&
-                    vec_ok(a->draft_logits, a->dtype, V, k, a->draft_stride_b, a->draft_stride_k);
-    if (launch_residual(a->dtype, vt, a->target_logits, a->target_stride_b, a->target_stride_k, a->draft_logits,
-                        a->draft_stride_b, a->draft_stride_k, B, k, V, w.plans, w.first_rej, a->u_resample,
-                        a->tokens, s) != hipSuccess)
-      return LPS_ELAUNCH;
+  const SpecOut out{a->n_accepted, a->tokens, a->accept, a->p_target, a->q_draft};
+  if (!lev) {
+    hipLaunchKernelGGL(spec_epilogue_kernel, dim3((B + 255) / 256), dim3(256), 0, s, B, k, a->temperature, w.p_t,
+                       w.q_d, w.draws_t, a->draft_tokens, a->u_accept, out);
+    return hipGetLastError() == hipSuccess ? LPS_OK : LPS_ELAUNCH;
   }
+  ResParams Q{};
+  Q.tl = a->target_logits;
+  Q.tsb = a->target_stride_b;
+  Q.tsk = a->target_stride_k;
+  Q.dl = a->draft_logits;
+  Q.dsb = a->draft_stride_b;
+  Q.dsk = a->draft_stride_k;
+  Q.B = B;
+  Q.k = k;
+  Q.V = V;
+  Q.T = a->temperature;
+  Q.p_t = w.p_t;
+  Q.q_d = w.q_d;
+  Q.draws_t = w.draws_t;
+  Q.draft_tokens = a->draft_tokens;
+  Q.u_acc = a->u_accept;
+  Q.u_res = a->u_resample;
+  Q.cut = w.cut;
+  Q.ties = w.ties;
+  Q.status = P.row_status;
+  Q.rec = w.rec;
+  Q.rsum = w.rsum;
+  Q.count = w.count;
+  Q.o = out;
+  if (launch_residual(a->dtype, vec && vec_d, Q, s) != hipSuccess) return LPS_ELAUNCH;
   return LPS_OK;
 }
 

@@ -34,16 +34,6 @@ constexpr int GEN_WIN = 8192;           // ids per history-count window: a multi
 constexpr int NBINS = 2048;        // radix digit bins (11 bits)
 constexpr uint32_t kNegInfKey = 0x007FFFFFu;  // f2key(-inf)
 
-struct RowPlan {
-  float zmax;        // max scaled logit
-  float T;           // effective temperature (1 for greedy)
-  uint32_t key_lo;   // kept: key > key_lo, or key == key_lo and tie rank < n_tie
-  uint32_t n_tie;    // kNoTie = all ties at key_lo kept
-  uint64_t Zf;       // fixed-point mass of the kept set
-  int32_t greedy;
-  int32_t argmax;
-};
-
 struct KParams {
   const void* logits;
   int V, R, rows_inner;
@@ -76,7 +66,6 @@ struct KParams {
   float* kept_cut;
   int32_t* kept_ties;
   int32_t* kept_count;
-  RowPlan* plans;
   const int32_t* only_status;  // non-null: process only rows whose entry has LPS_ROW_DEFERRED (8) set
   int32_t* row_path;           // optional: 0 fast kernel, 1 general kernel
   const uint32_t* allowed;     // optional legality bits, row r at allowed + r * allowed_stride
@@ -816,12 +805,6 @@ __device__ __forceinline__ void gen_row(const KParams& P, const int r, GenShared
     if (P.kept_ties) P.kept_ties[r] = n_tie == kNoTie ? -1 : (int32_t)n_tie;
     if (P.kept_count) P.kept_count[r] = (int32_t)kept_n;
     if (P.row_path) P.row_path[r] = 1;
-    if (P.plans) {
-      RowPlan pl;
-      pl.zmax = zmax; pl.T = Te; pl.key_lo = key_lo; pl.n_tie = n_tie; pl.Zf = Zf;
-      pl.greedy = greedy ? 1 : 0; pl.argmax = argmax;
-      P.plans[r] = pl;
-    }
   }
 }
 

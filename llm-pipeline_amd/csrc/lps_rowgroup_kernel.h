@@ -1598,7 +1598,8 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
       const uint32_t kq = f2key(zq);
       const bool kept = zq != -INFINITY && ((!nuc && tcase != TYP_LOW) || kq > vkey ||
                                             (kq == vkey && (n_tie == kNoTie || qtok <= tie_lim)));
-      if (kept) qprob = (float)((double)zmass_fix(zq, Rref) / (double)Zkept);
+      // (in the row mass's arithmetic, so that the rounding of c cancels against Z's)
+      if (kept) qprob = XF && targ ? 1.0f : (float)((double)emass(xq, c, Rref) * kFix / (double)Zkept);
     }
   }
   if (row_skips_draw(P, r) && !greedy) token = -1;

@@ -574,3 +574,43 @@ def test_spec_verify_first_token_law(dev, residual):
     _print(f"spec verify first-token law ({residual}): bins={int(big.sum())}+1 stat={stat:.1f} p={pval:.3g}; "
            f"other law p={p_other:.3g}")
     assert pval > 1e-4 and p_other < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,top_p,step", [(64, 0.9, 0.0), (4096, 1.0, 0.0), (4097, 0.95, 0.5), (8200, 0.9, 0.25),
+                                          (12289, 1.0, 0.0), (151936, 0.95, 0.0)])
+def test_leviathan_residual_chunks(dev, dtype, V, top_p, step):
+    """The residual draw at its chunk edges (4096 ids a workgroup), odd rows, and
+    logits rounded to ``step``, so that the top-p cut falls inside ties spread
+    over the chunks: the drawn id's interval of the cumulative residual (fp64,
+    vocabulary order, kept sets by a stable sort) holds u times the total, up to
+    2e-6 of it (fp32 masses of both rows)."""
+    from lps import spec_verify
+    B, k, T = 4, 2, 0.8
+    sw = W.c4(B=B, k=k, V=V, seed=V, temperature=T, top_p=top_p)
+    rnd = (lambda t: (t / step).round() * step) if step else (lambda t: t)
+    t, d = rnd(sw.target).to(dtype), rnd(sw.draft).to(dtype)
+    tok = d.float().argmax(-1)                      # likely drafts, rejected by a high uniform
+    ua = 0.9 + 0.0999 * sw.u_accept
+    out = spec_verify(t.to(dev), d.to(dev), tok.to(dev), ua.to(dev), sw.u_resample.to(dev), T, top_p,
+                      residual="leviathan")
+
+    def kept(x):
+        z = (x.float() / T).double().numpy()
+        order, _, n = O.top_p_truth(torch.from_numpy(z), top_p) if top_p < 1 else (np.arange(V), None, V)
+        e = np.zeros(V)
+        e[order[:n]] = np.exp(z[order[:n]] - z.max())
+        return e / e.sum()
+
+    drawn = 0
+    for b in range(B):
+        j = int(out.n_accepted[b])
+        if j == k:
+            continue
+        r = np.maximum(kept(t[b, j]) - kept(d[b, j]), 0.0)
+        cum = np.cumsum(r)
+        got, u = int(out.tokens[b, j]), float(sw.u_resample[b, j]) * cum[-1]
+        assert r[got] > 0
+        assert cum[got] - r[got] - 2e-6 * cum[-1] <= u <= cum[got] + 2e-6 * cum[-1], (b, j, got)
+        drawn += 1
+    assert drawn > 0
