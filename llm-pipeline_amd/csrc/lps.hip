@@ -390,21 +390,39 @@ size_t softmax_records_bytes(int rows, int G) {
   return G > 1 ? (size_t)rows * G * sizeof(SmRecord) + ((size_t)rows * 4 + 255) / 256 * 256 : 0;
 }
 
-template <int DT>
+// Columns a misaligned row is planned for: from its first 16-byte line.
+int softmax_span(int dtype, int cols) { return cols <= 0x7FFFFFFF - 7 ? cols + (dtype == LPS_DTYPE_F32 ? 3 : 7) : cols; }
+
+template <int DT, bool MA>
 hipError_t launch_softmax_reg(const SoftmaxParams& S, const SmPlan& p, hipStream_t s) {
   if (p.kind == 0) {
     const dim3 grid((S.rows + SM_NT / 64 - 1) / (SM_NT / 64));
     switch (p.nv) {
-      case 1: hipLaunchKernelGGL((softmax_wave_kernel<DT, 1>), grid, dim3(SM_NT), 0, s, S); break;
-      case 2: hipLaunchKernelGGL((softmax_wave_kernel<DT, 2>), grid, dim3(SM_NT), 0, s, S); break;
-      case 4: hipLaunchKernelGGL((softmax_wave_kernel<DT, 4>), grid, dim3(SM_NT), 0, s, S); break;
-      default: hipLaunchKernelGGL((softmax_wave_kernel<DT, 8>), grid, dim3(SM_NT), 0, s, S); break;
+      case 1: hipLaunchKernelGGL((softmax_wave_kernel<DT, 1, MA>), grid, dim3(SM_NT), 0, s, S); break;
+      case 2: hipLaunchKernelGGL((softmax_wave_kernel<DT, 2, MA>), grid, dim3(SM_NT), 0, s, S); break;
+      case 4: hipLaunchKernelGGL((softmax_wave_kernel<DT, 4, MA>), grid, dim3(SM_NT), 0, s, S); break;
+      default: hipLaunchKernelGGL((softmax_wave_kernel<DT, 8, MA>), grid, dim3(SM_NT), 0, s, S); break;
     }
   } else {
     const dim3 grid((unsigned)(((int64_t)S.rows + 7) / 8 * S.G * 8));
-    if (p.nv == 4) hipLaunchKernelGGL((softmax_chunk_kernel<DT, 4>), grid, dim3(SM_NT), 0, s, S);
-    else hipLaunchKernelGGL((softmax_chunk_kernel<DT, 8>), grid, dim3(SM_NT), 0, s, S);
+    if (p.nv == 4) hipLaunchKernelGGL((softmax_chunk_kernel<DT, 4, MA>), grid, dim3(SM_NT), 0, s, S);
+    else hipLaunchKernelGGL((softmax_chunk_kernel<DT, 8, MA>), grid, dim3(SM_NT), 0, s, S);
   }
+  return hipGetLastError();
+}
+template <int DT>
+hipError_t launch_softmax_reg(const SoftmaxParams& S, const SmPlan& p, bool ma, hipStream_t s) {
+  return ma ? launch_softmax_reg<DT, true>(S, p, s) : launch_softmax_reg<DT, false>(S, p, s);
+}
+
+// One streaming pass from the block statistics: nv vectors per lane.
+template <int DT>
+hipError_t launch_softmax_apply(const SoftmaxParams& S, int nv, bool ma, hipStream_t s) {
+  const dim3 grid((unsigned)(((int64_t)S.rows + 7) / 8 * S.G * 8));
+  if (nv == 8 && ma) hipLaunchKernelGGL((softmax_apply_kernel<DT, 8, true>), grid, dim3(SM_NT), 0, s, S);
+  else if (nv == 8) hipLaunchKernelGGL((softmax_apply_kernel<DT, 8, false>), grid, dim3(SM_NT), 0, s, S);
+  else if (ma) hipLaunchKernelGGL((softmax_apply_kernel<DT, 2, true>), grid, dim3(SM_NT), 0, s, S);
+  else hipLaunchKernelGGL((softmax_apply_kernel<DT, 2, false>), grid, dim3(SM_NT), 0, s, S);
   return hipGetLastError();
 }
 
@@ -791,8 +809,14 @@ int lps_verify_drafts(const void* target_probs, int32_t dtype, int64_t K, int64_
 
 size_t lps_softmax_workspace_bytes(int rows, int cols, int dtype) {
   if (rows <= 0 || cols < 1 || !dtype_ok(dtype)) return 0;
-  const SmPlan p = softmax_plan(dtype, rows, cols);
-  return p.kind == 1 ? softmax_records_bytes(rows, p.G) : 0;
+  // (aligned and misaligned rows may be planned apart)
+  size_t most = 0;
+  for (const int c : {cols, softmax_span(dtype, cols)}) {
+    const SmPlan p = softmax_plan(dtype, rows, c);
+    const size_t n = p.kind == 1 ? softmax_records_bytes(rows, p.G) : 0;
+    most = n > most ? n : most;
+  }
+  return most;
 }
 
 int lps_lm_head(const lps_lm_head_args* a, void* stream) {
@@ -847,44 +871,41 @@ int lps_softmax(const lps_softmax_args* a, void* stream) {
   S.row_lse = a->row_lse;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipError_t e;
-  // register-resident kernels: every row of x and out starts 16-byte aligned
-  const int vpl = a->dtype == LPS_DTYPE_F32 ? 4 : 8;
+  // register-resident kernels: every row of x and out starts 16-byte aligned,
+  // or every row of out is misaligned as its row of x is (mis)
+  const int vpl = a->dtype == LPS_DTYPE_F32 ? 4 : 8, es = 16 / vpl;
   auto aligned = [&](const void* p, int64_t stride) {
     return reinterpret_cast<uintptr_t>(p) % 16 == 0 && (a->rows <= 1 || stride % vpl == 0);
   };
+  const bool al = aligned(a->x, a->x_stride) && aligned(a->out, a->out_stride);
+  const bool mis = !al && reinterpret_cast<uintptr_t>(a->x) % es == 0 &&
+                   (reinterpret_cast<uintptr_t>(a->x) - reinterpret_cast<uintptr_t>(a->out)) % 16 == 0 &&
+                   (a->rows <= 1 || (a->x_stride - a->out_stride) % vpl == 0);
+  const int span = mis ? softmax_span(a->dtype, a->cols) : a->cols;
   if (a->row_stats) {
     // one streaming pass from the producer's block statistics
     const int nstats = a->stats_cols > 0 ? (int)(((int64_t)a->cols + a->stats_cols - 1) / a->stats_cols) : 0;
     if (a->causal || a->stats_cols < 1 || (a->rows > 1 && a->stats_stride < 2 * (int64_t)nstats)) return LPS_EINVAL;
-    if (aligned(a->x, a->x_stride) && aligned(a->out, a->out_stride)) {
-      const int64_t vecs = ((int64_t)a->cols + vpl - 1) / vpl;
+    if (al || mis) {
+      const int64_t vecs = ((int64_t)span + vpl - 1) / vpl;
       const int nv = vecs > (int64_t)SM_NT * 2 ? 8 : 2;
       S.G = (int)((vecs + (int64_t)SM_NT * nv - 1) / ((int64_t)SM_NT * nv));
       S.row_stats = a->row_stats;
       S.stats_stride = a->rows > 1 ? a->stats_stride : 2 * (int64_t)nstats;
       S.nstats = nstats;
-      const dim3 grid((unsigned)(((int64_t)S.rows + 7) / 8 * S.G * 8));
-#define SMA_LAUNCH(DT)                                                                       \
-  do {                                                                                       \
-    if (nv == 8) hipLaunchKernelGGL((softmax_apply_kernel<DT, 8>), grid, dim3(SM_NT), 0, s, S); \
-    else hipLaunchKernelGGL((softmax_apply_kernel<DT, 2>), grid, dim3(SM_NT), 0, s, S);         \
-  } while (0)
       switch (a->dtype) {
-        case LPS_DTYPE_F32: SMA_LAUNCH(LPS_DTYPE_F32); break;
-        case LPS_DTYPE_BF16: SMA_LAUNCH(LPS_DTYPE_BF16); break;
-        default: SMA_LAUNCH(LPS_DTYPE_F16); break;
+        case LPS_DTYPE_F32: e = launch_softmax_apply<LPS_DTYPE_F32>(S, nv, mis, s); break;
+        case LPS_DTYPE_BF16: e = launch_softmax_apply<LPS_DTYPE_BF16>(S, nv, mis, s); break;
+        default: e = launch_softmax_apply<LPS_DTYPE_F16>(S, nv, mis, s); break;
       }
-#undef SMA_LAUNCH
-      e = hipGetLastError();
       return e == hipSuccess ? LPS_OK : LPS_ELAUNCH;
     }
   }
-  if (aligned(a->x, a->x_stride) && aligned(a->out, a->out_stride)) {
-    SmPlan p = softmax_plan(a->dtype, a->rows, a->cols);
+  if (al || mis) {
+    SmPlan p = softmax_plan(a->dtype, a->rows, span);
     if (p.kind == 1 && p.G > 1) {
       // split rows need the workspace, and distinct input and output (a
       // workgroup that falls back re-reads its whole row)
-      const int es = a->dtype == LPS_DTYPE_F32 ? 4 : 2;
       const char* x0 = static_cast<const char*>(a->x);
       const char* o0 = static_cast<const char*>(a->out);
       const int64_t xs = a->rows > 1 ? a->x_stride : a->cols, os = a->rows > 1 ? a->out_stride : a->cols;
@@ -904,9 +925,9 @@ int lps_softmax(const lps_softmax_args* a, void* stream) {
     }
     if (p.kind != 2) {
       switch (a->dtype) {
-        case LPS_DTYPE_F32: e = launch_softmax_reg<LPS_DTYPE_F32>(S, p, s); break;
-        case LPS_DTYPE_BF16: e = launch_softmax_reg<LPS_DTYPE_BF16>(S, p, s); break;
-        default: e = launch_softmax_reg<LPS_DTYPE_F16>(S, p, s); break;
+        case LPS_DTYPE_F32: e = launch_softmax_reg<LPS_DTYPE_F32>(S, p, mis, s); break;
+        case LPS_DTYPE_BF16: e = launch_softmax_reg<LPS_DTYPE_BF16>(S, p, mis, s); break;
+        default: e = launch_softmax_reg<LPS_DTYPE_F16>(S, p, mis, s); break;
       }
       return e == hipSuccess ? LPS_OK : LPS_ELAUNCH;
     }

@@ -3,6 +3,14 @@
 // fused_softmax_triton; reference semantics at :105-113:
 // softmax(masked_fill(col > row + offset, -inf)) in fp32, out in the input dtype).
 //
+// Rows that do not start on 16 bytes (an odd number of columns) take the same
+// register kernels when a row's input and output are misaligned alike: the
+// row is walked from the 16-byte line that holds its first element, `mis`
+// elements before it, in whole aligned vectors; the elements of the first and
+// last vector that lie outside the row are neither read nor written.  128 x
+// 129 rows of 1601 bf16 columns, causal at offset 1472: 74.4 us on the
+// three-pass kernel, element by element.
+//
 // Three kernels, chosen per call by the host:
 //  * softmax_wave_kernel: one wave per row (rows of up to 64 x 32 words: 2048
 //    fp32 / 4096 16-bit columns).  The row is read once into registers, the
@@ -19,8 +27,8 @@
 //    and a workgroup that times out computes every chunk's record itself
 //    from the row (the same arithmetic, so the same result).
 //  * softmax_kernel: one workgroup per row in three passes (max; sum; output),
-//    for rows that are not 16-byte aligned, longer rows, calls without a
-//    workspace and in-place calls of split rows.
+//    for rows whose input and output are misaligned differently, longer rows,
+//    calls without a workspace and in-place calls of split rows.
 //
 // Arithmetic of the register kernels, per lane: m = the lane's max, then
 // e = exp2(fma(x, c, -m c)) (c = log2 e) replaces x in the registers, summed in
@@ -198,8 +206,9 @@ __device__ __forceinline__ MS block_reduce_ms(MS v, SmShared& sh) {
 // group's max times c, and returns the lane's pair; store() writes e times its
 // group's scale.  A group depends only on its own loads, so its exponentials
 // run while the loads of later groups are in flight.  FULL: the whole chunk
-// lies before lim and inside the row (no bounds checks).
-template <int DT, int NV, int LANES>
+// lies before lim and inside the row (no bounds checks).  MA: the row starts at
+// element mis of its first 16-byte line; row, base, lim and n count from there.
+template <int DT, int NV, int LANES, bool MA = false>
 struct RegChunk {
   static constexpr int VPL = DT == LPS_DTYPE_F32 ? 4 : 8;   // elements per 16 bytes
   static constexpr int GV = NV < 2 ? NV : 2;                // vectors per group (the last may hold 1)
@@ -212,7 +221,7 @@ struct RegChunk {
   __device__ __forceinline__ static int row0(int base, int k) { return base + k * LANES * VPL; }   // uniform
 
   template <bool FULL>
-  __device__ __forceinline__ void load(const void* row, int base, int lane, int lim) {
+  __device__ __forceinline__ void load(const void* row, int base, int lane, int lim, int mis = 0) {
 #pragma unroll
     for (int k = 0; k < NV; k++) {
       const int i0 = at(base, k, lane);
@@ -223,11 +232,12 @@ struct RegChunk {
       if (row0(base, k) >= lim) {
 #pragma unroll
         for (int e = 0; e < VPL; e++) v[k][e] = -INFINITY;
-      } else if (i0 + VPL <= lim) {
+      } else if ((!MA || i0 >= mis) && i0 + VPL <= lim) {
         loadv<DT, VPL>(row, i0, v[k]);
       } else {
 #pragma unroll
-        for (int e = 0; e < VPL; e++) v[k][e] = i0 + e < lim ? load1<DT>(row, i0 + e) : -INFINITY;
+        for (int e = 0; e < VPL; e++)
+          v[k][e] = (!MA || i0 + e >= mis) && i0 + e < lim ? load1<DT>(row, i0 + e) : -INFINITY;
       }
     }
   }
@@ -297,7 +307,7 @@ struct RegChunk {
 
   // writes e times exp2(mc_g - M c) / S for the row pair (M, S)
   template <bool FULL>
-  __device__ __forceinline__ void store(void* orow, int base, int lane, int n, MS row) const {
+  __device__ __forceinline__ void store(void* orow, int base, int lane, int n, MS row, int mis = 0) const {
     const float Mc = __fmul_rn(row.m, SM_LOG2E);
     const double inv = 1.0 / row.s;
 #pragma unroll
@@ -309,17 +319,34 @@ struct RegChunk {
         float p[VPL];
 #pragma unroll
         for (int e = 0; e < VPL; e++) p[e] = __fmul_rn(v[k][e], sc);
-        if (FULL || i0 + VPL <= n) {
+        if (FULL || ((!MA || i0 >= mis) && i0 + VPL <= n)) {
           store16<DT>(orow, i0, p);
         } else {
 #pragma unroll
           for (int e = 0; e < VPL; e++)
-            if (i0 + e < n) store1<DT>(orow, i0 + e, p[e]);
+            if ((!MA || i0 + e >= mis) && i0 + e < n) store1<DT>(orow, i0 + e, p[e]);
         }
       }
     }
   }
 };
+
+// Row r's first 16-byte line in the input and in the output (misaligned
+// alike, the host's check) and the row's first element in it.
+struct SmRow {
+  const void* x;
+  void* out;
+  int mis;
+};
+template <int DT, bool MA>
+__device__ __forceinline__ SmRow sm_row(const SoftmaxParams& S, int r) {
+  constexpr int ES = DT == LPS_DTYPE_F32 ? 4 : 2;
+  const char* row = reinterpret_cast<const char*>(S.x) + (int64_t)ES * r * S.x_stride;
+  char* orow = reinterpret_cast<char*>(S.out) + (int64_t)ES * r * S.out_stride;
+  if (!MA) return SmRow{row, orow, 0};
+  const int off = (int)(reinterpret_cast<uintptr_t>(row) & 15);
+  return SmRow{row - off, orow - off, off / ES};
+}
 
 // log(sum(exp(x))) of a row from its pair: -inf for an all -inf row, NaN for a
 // row holding a NaN or +inf.
@@ -328,28 +355,26 @@ __device__ __forceinline__ float row_lse_value(MS row) {
   return (float)((double)__fmul_rn(row.m, SM_LOG2E) * SM_LN2 + log(row.s));
 }
 
-template <int DT, int NV, bool FULL>
-__device__ __forceinline__ void wave_row(const SoftmaxParams& S, const void* row, void* orow, int r, int lane, int lim) {
-  RegChunk<DT, NV, 64> C;
-  C.template load<FULL>(row, 0, lane, lim);
-  const MS rs = wreduce_ms(C.template exps<FULL>(0, lim));
+template <int DT, int NV, bool FULL, bool MA>
+__device__ __forceinline__ void wave_row(const SoftmaxParams& S, const SmRow& q, int r, int lane, int lim) {
+  RegChunk<DT, NV, 64, MA> C;
+  C.template load<FULL>(q.x, 0, lane, lim + q.mis, q.mis);
+  const MS rs = wreduce_ms(C.template exps<FULL>(0, lim + q.mis));
   if (S.row_lse && lane == 0) S.row_lse[r] = row_lse_value(rs);
-  C.template store<FULL>(orow, 0, lane, S.cols, rs);
+  C.template store<FULL>(q.out, 0, lane, S.cols + q.mis, rs, q.mis);
 }
 
 // One wave per row.
-template <int DT, int NV>
+template <int DT, int NV, bool MA>
 __global__ __launch_bounds__(SM_NT) void softmax_wave_kernel(SoftmaxParams S) {
   const int r = blockIdx.x * (SM_NT / 64) + (threadIdx.x >> 6);
   if (r >= S.rows) return;   // whole waves leave; no block barrier follows
-  constexpr int ES = DT == LPS_DTYPE_F32 ? 4 : 2;
   constexpr int CH = 64 * NV * RegChunk<DT, NV, 64>::VPL;
   const int lane = threadIdx.x & 63;
-  const void* row = reinterpret_cast<const char*>(S.x) + (int64_t)ES * r * S.x_stride;
-  void* orow = reinterpret_cast<char*>(S.out) + (int64_t)ES * r * S.out_stride;
+  const SmRow q = sm_row<DT, MA>(S, r);
   const int lim = causal_limit(S, r);
-  if (lim == CH && S.cols == CH) wave_row<DT, NV, true>(S, row, orow, r, lane, lim);
-  else wave_row<DT, NV, false>(S, row, orow, r, lane, lim);
+  if (!MA && lim == CH && S.cols == CH) wave_row<DT, NV, true, false>(S, q, r, lane, lim);
+  else wave_row<DT, NV, false, MA>(S, q, r, lane, lim);
 }
 
 __device__ __forceinline__ uint32_t l2_add_u32(uint32_t* p, uint32_t v) {
@@ -368,16 +393,18 @@ __device__ __forceinline__ MS unpack_record(unsigned long long w) {
 // Chunk j of row r.  With G > 1: publish the chunk's record, wait for the
 // row's others (or fall back to the row), store, then count this workgroup
 // out of the row's records.
-template <int DT, int NV, bool FULL>
-__device__ __forceinline__ void chunk_row(const SoftmaxParams& S, SmShared& sh, const void* row, void* orow, int r,
-                                          int j, int lim) {
-  using RC = RegChunk<DT, NV, SM_NT>;
+template <int DT, int NV, bool FULL, bool MA>
+__device__ __forceinline__ void chunk_row(const SoftmaxParams& S, SmShared& sh, const SmRow& q, int r, int j, int lim) {
+  using RC = RegChunk<DT, NV, SM_NT, MA>;
+  const void* row = q.x;
+  void* orow = q.out;
+  lim += q.mis;
   constexpr int CH = SM_NT * NV * RC::VPL;
   const int G = S.G;
   const int tid = threadIdx.x;
   const int base = j * CH;
   RC C;
-  C.template load<FULL>(row, base, tid, lim);
+  C.template load<FULL>(row, base, tid, lim, q.mis);
   const MS ch = block_reduce_ms(C.template exps<FULL>(base, lim), sh);
   MS rs = ch;
   unsigned long long* rec = reinterpret_cast<unsigned long long*>(S.records) + (int64_t)r * G;
@@ -414,7 +441,7 @@ __device__ __forceinline__ void chunk_row(const SoftmaxParams& S, SmShared& sh, 
       // the host never splits an in-place call)
       unsigned long long w = 0ull;
       for (int t = 0; t < G; t++) {
-        C.template load<false>(row, t * CH, tid, lim);
+        C.template load<false>(row, t * CH, tid, lim, q.mis);
         const MS ct = block_reduce_ms(C.template exps<false>(t * CH, lim), sh);
         if (tid == t) w = pack_record(ct);
       }
@@ -425,14 +452,14 @@ __device__ __forceinline__ void chunk_row(const SoftmaxParams& S, SmShared& sh, 
           sh.S = row_pair.s;
         }
       }
-      C.template load<FULL>(row, base, tid, lim);
+      C.template load<FULL>(row, base, tid, lim, q.mis);
       C.template exps<FULL>(base, lim);
       __syncthreads();
     }
     rs = MS{sh.M, sh.S};
   }
   if (S.row_lse && j == 0 && tid == 0) S.row_lse[r] = row_lse_value(rs);
-  C.template store<FULL>(orow, base, tid, S.cols, rs);
+  C.template store<FULL>(orow, base, tid, S.cols + q.mis, rs, q.mis);
   if (G > 1 && tid < 64) {
     // this workgroup reads no record any more; the row's last one zeroes the
     // row's records and counter for the next launch
@@ -447,20 +474,18 @@ __device__ __forceinline__ void chunk_row(const SoftmaxParams& S, SmShared& sh, 
 
 // G workgroups per row (workgroup b: XCD b % 8, row (b / 8) / G * 8 + b % 8,
 // chunk (b / 8) % G), each holding CH = 256 * NV * VPL columns in registers.
-template <int DT, int NV>
+template <int DT, int NV, bool MA>
 __global__ __launch_bounds__(SM_NT) void softmax_chunk_kernel(SoftmaxParams S) {
   __shared__ SmShared sh;
-  constexpr int ES = DT == LPS_DTYPE_F32 ? 4 : 2;
   constexpr int CH = SM_NT * NV * RegChunk<DT, NV, SM_NT>::VPL;
   const int G = S.G;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int r = (slot / G) * 8 + xcd, j = slot % G;
   if (r >= S.rows) return;   // uniform over the workgroup
-  const void* row = reinterpret_cast<const char*>(S.x) + (int64_t)ES * r * S.x_stride;
-  void* orow = reinterpret_cast<char*>(S.out) + (int64_t)ES * r * S.out_stride;
+  const SmRow q = sm_row<DT, MA>(S, r);
   const int lim = causal_limit(S, r);
-  if ((j + 1) * CH <= lim) chunk_row<DT, NV, true>(S, sh, row, orow, r, j, lim);   // lim <= cols
-  else chunk_row<DT, NV, false>(S, sh, row, orow, r, j, lim);
+  if (!MA && (j + 1) * CH <= lim) chunk_row<DT, NV, true, false>(S, sh, q, r, j, lim);   // lim <= cols
+  else chunk_row<DT, NV, false, MA>(S, sh, q, r, j, lim);
 }
 
 // Single pass from block statistics (the LM-head epilogue's): every
@@ -468,10 +493,9 @@ __global__ __launch_bounds__(SM_NT) void softmax_chunk_kernel(SoftmaxParams S) {
 // order (thread t takes pairs t, t + 256, ...; then the block reduction), so
 // all of them hold the same (M, S); then its chunk is streamed as
 // exp2(x c - M c) / S.  Mapping as the chunk kernel's.
-template <int DT, int NV>
+template <int DT, int NV, bool MA>
 __global__ __launch_bounds__(SM_NT) void softmax_apply_kernel(SoftmaxParams S) {
   __shared__ SmShared sh;
-  constexpr int ES = DT == LPS_DTYPE_F32 ? 4 : 2;
   constexpr int VPL = DT == LPS_DTYPE_F32 ? 4 : 8;
   constexpr int CH = SM_NT * NV * VPL;
   const int G = S.G;
@@ -479,19 +503,21 @@ __global__ __launch_bounds__(SM_NT) void softmax_apply_kernel(SoftmaxParams S) {
   const int r = (slot / G) * 8 + xcd, j = slot % G;
   if (r >= S.rows) return;   // uniform over the workgroup
   const int tid = threadIdx.x;
-  const void* row = reinterpret_cast<const char*>(S.x) + (int64_t)ES * r * S.x_stride;
-  void* orow = reinterpret_cast<char*>(S.out) + (int64_t)ES * r * S.out_stride;
-  const int n = S.cols;
+  const SmRow q = sm_row<DT, MA>(S, r);
+  const void* row = q.x;
+  void* orow = q.out;
+  const int n = S.cols + q.mis, mis = q.mis;
   // the chunk's loads first: they are in flight while the statistics combine
   float v[NV][VPL];
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     const int i0 = j * CH + (k * SM_NT + tid) * VPL;
-    if (i0 + VPL <= n) {
+    if ((!MA || i0 >= mis) && i0 + VPL <= n) {
       loadv<DT, VPL>(row, i0, v[k]);
     } else {
 #pragma unroll
-      for (int e = 0; e < VPL; e++) v[k][e] = i0 + e < n ? load1<DT>(row, i0 + e) : -INFINITY;
+      for (int e = 0; e < VPL; e++)
+        v[k][e] = (!MA || i0 + e >= mis) && i0 + e < n ? load1<DT>(row, i0 + e) : -INFINITY;
     }
   }
   const float* st = S.row_stats + (int64_t)r * S.stats_stride;
@@ -508,12 +534,12 @@ __global__ __launch_bounds__(SM_NT) void softmax_apply_kernel(SoftmaxParams S) {
     float p[VPL];
 #pragma unroll
     for (int e = 0; e < VPL; e++) p[e] = __fmul_rn(__builtin_amdgcn_exp2f(__builtin_fmaf(v[k][e], SM_LOG2E, -Mc)), inv);
-    if (i0 + VPL <= n) {
+    if ((!MA || i0 >= mis) && i0 + VPL <= n) {
       store16<DT>(orow, i0, p);
     } else {
 #pragma unroll
       for (int e = 0; e < VPL; e++)
-        if (i0 + e < n) store1<DT>(orow, i0 + e, p[e]);
+        if ((!MA || i0 + e >= mis) && i0 + e < n) store1<DT>(orow, i0 + e, p[e]);
     }
   }
 }

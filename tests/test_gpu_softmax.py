@@ -242,3 +242,27 @@ def test_softmax_workspace_reuse_across_layouts(dev):
         _check(out, x)
         for t in SM._WS.values():
             assert int(t.count_nonzero()) == 0, f"{shape} {dtype}: records left in the workspace"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols", [(9, 1), (33, 255), (21, 505), (8, 513), (16, 2041), (5, 4089), (6, 4097), (3, 8187),
+                                       (2, 16379), (9, 16385), (4, 100001)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_softmax_rows_off_the_16_byte_lines(dev, dtype, rows, cols, causal):
+    """Odd row lengths (every row starts elsewhere in its 16-byte line) at the
+    edges of the wave and chunk plans, whose span counts from that line, and the
+    elements beside the rows left alone; _check's bounds."""
+    g = torch.Generator().manual_seed(rows * cols)
+    x = (torch.randn((rows, cols), generator=g) * 4.0).to(dtype)
+    off = max(0, cols - rows)
+    out, lse = fused_softmax(x.to(dev), causal=causal, row_offset=off, return_lse=True)
+    _check(out, x, causal=causal, row_offset=off)
+    xd = x.double()
+    if causal:
+        xd = xd.masked_fill(torch.arange(cols).unsqueeze(0) > torch.arange(rows).unsqueeze(1) + off, float("-inf"))
+    torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(xd, dim=-1), atol=1e-5, rtol=1e-6)
+    big = torch.full((rows * cols + 8,), 7.0, dtype=dtype, device=dev)     # rows from the second element on
+    big[1:1 + rows * cols] = x.to(dev).reshape(-1)
+    out = fused_softmax(big[1:1 + rows * cols].view(rows, cols), causal=causal, row_offset=off)
+    _check(out, x, causal=causal, row_offset=off)
+    assert bool((big[:1] == 7).all()) and bool((big[1 + rows * cols:] == 7).all())
