@@ -3,6 +3,8 @@ pointers, the current HIP stream and per-row parameter tensors."""
 
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from . import _lib
@@ -34,7 +36,28 @@ def ptr(t) -> int:
 
 
 def stream_of(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """The device's current stream as an integer handle (the raw accessor: a
+    ``torch.cuda.Stream`` object costs 2.5 us a call, this 0.2)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+_NO_GUARD = contextlib.nullcontext()
+
+
+def guard(device: torch.device):
+    """Makes ``device`` current for a launch; nothing to do (and to undo) when it is."""
+    return _NO_GUARD if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+
+
+def on(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """``t`` on ``device`` as ``dtype`` (``t`` itself when it is)."""
+    return t if t.dtype is dtype and t.device == device else t.to(device=device, dtype=dtype)
+
+
+def flat(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """``t`` on ``device`` as a contiguous vector of ``dtype``."""
+    t = on(t, device, dtype)
+    return t if t.dim() == 1 and t.is_contiguous() else t.reshape(-1).contiguous()
 
 
 def as_f32(v, B: int, device) -> torch.Tensor:

@@ -131,6 +131,8 @@ _lock = threading.Lock()
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Load (once) and type the shared library; raises if it is not built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

@@ -9,6 +9,7 @@ once per row (``src/llm_pipeline/inference/continuous_batching.py:394-401``);
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from dataclasses import dataclass, fields
 from typing import Iterable, Optional, Sequence
@@ -77,13 +78,19 @@ def workspace_for(device: torch.device, nbytes: int) -> torch.Tensor:
     Every launch leaves it ready for the next, so it is filled only when it is
     created; launches on one stream never overlap, so they may share it."""
     dev = torch.device(device)
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    key = (dev.index, D.stream_of(dev))
     with _WS_LOCK:
         t = _WS.get(key)
         if t is None or t.numel() < nbytes:
             t = torch.zeros((max(nbytes, 1 << 20),), dtype=torch.uint8, device=dev)
             _WS[key] = t
         return t
+
+
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(device_index: int, B: int, V: int, flags: int) -> int:
+    """``lps_workspace_bytes`` on the current device, a function of the sizes alone."""
+    return _lib.load().lps_workspace_bytes(B, V, flags)
 
 
 @dataclass
@@ -111,6 +118,16 @@ def row_kind_flags(temperature, top_k, min_p=None, typical_p=None) -> int:
     whose values the host does not hold.  The hints only choose which kernels
     (and which build of the row-group kernel) a launch runs; a row that breaks
     one is still sampled exactly, by the general kernel."""
+    if all(isinstance(v, (int, float)) for v in (temperature, top_k)) and \
+            all(v is None or isinstance(v, (int, float)) for v in (min_p, typical_p)):
+        # one row's values: the rule below without tensors (their construction
+        # costs a single-request call 12 us)
+        flags = 0
+        if min_p is not None and typical_p is not None and not (min_p > 0 or typical_p < 1 or top_k > FAST_KMAX):
+            flags |= _lib.LPS_FLAG_ROWS_BASIC_FILTERS
+        topk_row = not temperature > 0 or top_k > 0
+        return flags | (_lib.LPS_FLAG_ROWS_TOPK if topk_row else _lib.LPS_FLAG_ROWS_NUCLEUS)
+
     def host(v):
         if isinstance(v, torch.Tensor):
             return v.reshape(-1) if v.device.type == "cpu" else None
@@ -229,7 +246,7 @@ def sample_rows(logits: torch.Tensor, params: SamplingParams, uniforms: Optional
     if uniforms is None and not skip_draw:
         uniforms = torch.rand((B,), device=dev, dtype=torch.float32, generator=generator)
     if uniforms is not None:
-        uniforms = uniforms.to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+        uniforms = D.flat(uniforms, dev, torch.float32)
         if uniforms.numel() != B:
             raise ValueError("uniforms must hold one value per row")
     tokens = torch.empty((B,), dtype=torch.int64, device=dev)
@@ -248,7 +265,7 @@ def sample_rows(logits: torch.Tensor, params: SamplingParams, uniforms: Optional
         out.kept_ties = torch.empty((B,), dtype=torch.int32, device=dev)
         out.kept_count = torch.empty((B,), dtype=torch.int32, device=dev)
     if query_tokens is not None:
-        query_tokens = query_tokens.to(device=dev, dtype=torch.int64).reshape(-1).contiguous()
+        query_tokens = D.flat(query_tokens, dev, torch.int64)
         out.query_prob = torch.empty((B,), dtype=torch.float32, device=dev)
     if append_history:
         if histories is None or history_lengths is None:
@@ -259,14 +276,14 @@ def sample_rows(logits: torch.Tensor, params: SamplingParams, uniforms: Optional
             raise ValueError("append_history writes the histories in place: they must be int32 tensors on "
                              "the logits' device (row-contiguous [B, H], contiguous lengths [B])")
     if histories is not None:
-        histories = histories.to(device=dev, dtype=torch.int32)
+        histories = D.on(histories, dev, torch.int32)
         if histories.dim() != 2 or histories.shape[0] != B:
             raise ValueError("histories must be int32 [B, H]")
         if histories.stride(1) != 1:
             histories = histories.contiguous()
         if history_lengths is None:
             history_lengths = torch.full((B,), histories.shape[1], dtype=torch.int32, device=dev)
-        history_lengths = history_lengths.to(device=dev, dtype=torch.int32).contiguous()
+        history_lengths = D.on(history_lengths, dev, torch.int32).contiguous()
     if allowed is not None:
         if allowed.dtype == torch.bool:
             if tuple(allowed.shape) != (B, V):
@@ -277,60 +294,35 @@ def sample_rows(logits: torch.Tensor, params: SamplingParams, uniforms: Optional
             if allowed.dim() != 2 or allowed.shape[0] != B or allowed.shape[1] < (V + 31) // 32:
                 raise ValueError(f"allowed bits must be int32 [{B}, >= {(V + 31) // 32}]")
             allowed = allowed.contiguous()
-    p = params
-    a = _lib.SampleArgs()
-    a.logits = D.ptr(logits)
-    a.dtype = dt
-    a.num_rows = B
-    a.vocab = V
-    a.rows_inner = 1
-    a.stride_outer = logits.stride(0)
-    a.stride_inner = 0
-    a.temperature = D.ptr(p.temperature)
-    a.top_k = D.ptr(p.top_k)
-    a.top_p = D.ptr(p.top_p)
-    a.min_p = D.ptr(p.min_p)
-    a.typical_p = D.ptr(p.typical_p)
-    a.repetition_penalty = D.ptr(p.repetition_penalty)
-    a.presence_penalty = D.ptr(p.presence_penalty)
-    a.frequency_penalty = D.ptr(p.frequency_penalty)
-    a.history = D.ptr(histories)
-    a.history_stride = histories.stride(0) if histories is not None else 0
-    a.history_len = D.ptr(history_lengths) if histories is not None else 0
-    a.uniforms = D.ptr(uniforms)
-    a.query_tokens = D.ptr(query_tokens)
-    a.query_inner = 1 if query_tokens is not None else 0
-    a.query_prob = D.ptr(out.query_prob)
-    a.tokens = D.ptr(tokens)
-    a.chosen_logprob = D.ptr(out.chosen_logprob)
-    a.top_logprobs = D.ptr(out.top_logprobs)
-    a.top_ids = D.ptr(out.top_ids)
-    a.n_top = top_logprobs
-    a.entropy = D.ptr(out.entropy)
-    a.row_status = D.ptr(status)
-    a.skip_draw = 1 if skip_draw else 0
-    a.kept_cut = D.ptr(out.kept_cut)
-    a.kept_ties = D.ptr(out.kept_ties)
-    a.kept_count = D.ptr(out.kept_count)
-    a.row_path = D.ptr(out.row_path)
     hints = _lib.LPS_FLAG_ROWS_TOPK | _lib.LPS_FLAG_ROWS_NUCLEUS | _lib.LPS_FLAG_ROWS_BASIC_FILTERS
     if row_kind_hint & ~hints:
         raise ValueError("row_kind_hint takes LPS_FLAG_ROWS_TOPK / LPS_FLAG_ROWS_NUCLEUS / "
                          "LPS_FLAG_ROWS_BASIC_FILTERS only")
-    a.flags = ((0 if path == "auto" else _lib.LPS_FLAG_GENERIC) | (_lib.LPS_FLAG_APPEND_HISTORY if append_history else 0)
-               | row_kind_hint)
-    if noalloc:
-        a.workspace = 0
-        a.workspace_bytes = 0
-    else:
-        ws_bytes = _lib.load().lps_workspace_bytes(B, V, a.flags)
-        ws = workspace_for(dev, ws_bytes) if ws_bytes else None
-        a.workspace = D.ptr(ws)
-        a.workspace_bytes = ws.numel() if ws is not None else 0
-    a.allowed = D.ptr(allowed)
-    a.allowed_stride = allowed.stride(0) if allowed is not None else 0
-    entry = "lps_sample_noalloc" if noalloc else "lps_sample"
-    with torch.cuda.device(dev):
+    flags = ((0 if path == "auto" else _lib.LPS_FLAG_GENERIC) | (_lib.LPS_FLAG_APPEND_HISTORY if append_history else 0)
+             | row_kind_hint)
+    p, ptr = params, D.ptr
+    with D.guard(dev):
+        ws = None
+        if not noalloc:
+            ws_bytes = _workspace_bytes(dev.index, B, V, flags)
+            ws = workspace_for(dev, ws_bytes) if ws_bytes else None
+        # (in the order of the structure's fields)
+        a = _lib.SampleArgs(
+            ptr(logits), dt, B, V, 1, logits.stride(0), 0,
+            ptr(p.temperature), ptr(p.top_k), ptr(p.top_p), ptr(p.min_p), ptr(p.typical_p),
+            ptr(p.repetition_penalty), ptr(p.presence_penalty), ptr(p.frequency_penalty),
+            ptr(histories), 0 if histories is None else histories.stride(0),
+            0 if histories is None else ptr(history_lengths),
+            ptr(uniforms),
+            ptr(query_tokens), 0 if query_tokens is None else 1, ptr(out.query_prob),
+            ptr(tokens), ptr(out.chosen_logprob), ptr(out.top_logprobs), ptr(out.top_ids), top_logprobs,
+            ptr(out.entropy), ptr(status), 1 if skip_draw else 0,
+            ptr(out.kept_cut), ptr(out.kept_ties), ptr(out.kept_count),
+            ptr(out.row_path),
+            flags,
+            ptr(ws), 0 if ws is None else ws.numel(),
+            ptr(allowed), 0 if allowed is None else allowed.stride(0))
+        entry = "lps_sample_noalloc" if noalloc else "lps_sample"
         rc = getattr(_lib.load(), entry)(ctypes.byref(a), D.stream_of(dev))
     _lib.check(rc, entry)
     return out
@@ -339,7 +331,6 @@ def sample_rows(logits: torch.Tensor, params: SamplingParams, uniforms: Optional
 def raise_on_status(status: torch.Tensor) -> None:
     """Raise what the reference raises for rows the kernel could not sample
     (``torch.multinomial`` rejects NaN / inf / empty distributions)."""
-    bad = int(status.ne(0).any().item())
-    if not bad:
+    if not any(status.reshape(-1).tolist()):   # (one copy; a reduction on the device is two launches more)
         return
     raise RuntimeError("probability tensor contains either `inf`, `nan` or element < 0")

@@ -55,7 +55,7 @@ def lm_head(hidden: torch.Tensor, weight: torch.Tensor, out_dtype: Optional[torc
     a.w_stride = w.stride(0)
     a.out_stride = V
     if M:
-        with torch.cuda.device(hidden.device):
+        with D.guard(hidden.device):
             rc = _lib.load().lps_lm_head(ctypes.byref(a), D.stream_of(hidden.device))
         _lib.check(rc, "lps_lm_head")
     out = out.reshape(*lead, V)

@@ -16,6 +16,7 @@ arguments to ``sample_token``.
 from __future__ import annotations
 
 import math
+from array import array
 from dataclasses import dataclass
 from typing import Any, Dict, List, Optional
 
@@ -53,12 +54,51 @@ _CONFIG_KEYS = (
 )
 
 
+def _upload_history(ids: List[int], B: int, dev: torch.device) -> tuple:
+    """One history for every row: ``int32 [B, n]`` and lengths ``int32 [B]`` on
+    the device, in one copy (from pinned memory, which does not wait for the
+    stream, unless a graph is being captured)."""
+    try:
+        h = torch.frombuffer(array("i", ids), dtype=torch.int32)
+    except (TypeError, OverflowError):   # (what torch converts or rejects)
+        h = torch.tensor(list(ids), dtype=torch.int32)
+    n = h.numel()
+    pin = not torch.cuda.is_current_stream_capturing()
+    buf = torch.empty((n + B,), dtype=torch.int32, pin_memory=pin)
+    buf[:n] = h
+    buf[n:] = n
+    buf = buf.to(dev, non_blocking=pin)
+    return buf[:n].unsqueeze(0).expand(B, n).contiguous(), buf[n:]
+
+
 class Sampler:
     """Centralised logits -> token sampler on MI355X."""
+
+    _PARAM_SETS = 8   # shared parameter tensors kept per sampler
 
     def __init__(self, config: Optional[SamplingConfig] = None):
         self.config = config or SamplingConfig()
         self.last_output = None
+        self._params = {}
+
+    def _shared_params(self, B: int, dev: torch.device, config: "SamplingConfig") -> SamplingParams:
+        """The config's values for every row as device tensors: 8 fills a call
+        when built each time, so the last few sets are kept, by the values they
+        hold, the rows and the stream that filled them.  A call under graph
+        capture builds its own (a graph's tensors are the graph's, and a kept
+        set may be dropped while the graph lives)."""
+        values = (config.temperature, config.top_k, config.top_p, config.min_p, config.typical_p,
+                  config.repetition_penalty, config.presence_penalty, config.frequency_penalty)
+        if not all(isinstance(v, (int, float)) and v == v for v in values) or \
+                torch.cuda.is_current_stream_capturing():
+            return SamplingParams.build(B, dev, *values)
+        key = (B, dev.index, D.stream_of(dev), values)
+        p = self._params.get(key)
+        if p is None:
+            if len(self._params) >= self._PARAM_SETS:
+                self._params.clear()
+            p = self._params[key] = SamplingParams.build(B, dev, *values)
+        return p
 
     def sample_token(self, logits: torch.Tensor, config_override: Optional[Dict[str, Any]] = None,
                      generated_tokens: Optional[List[int]] = None, *, uniforms: Optional[torch.Tensor] = None,
@@ -94,14 +134,9 @@ class Sampler:
         hint = 0
         if params is None:
             hint = row_kind_flags(config.temperature, config.top_k, config.min_p, config.typical_p)
-            params = SamplingParams.build(
-                B, dev, temperature=config.temperature, top_k=config.top_k, top_p=config.top_p,
-                min_p=config.min_p, typical_p=config.typical_p, repetition_penalty=config.repetition_penalty,
-                presence_penalty=config.presence_penalty, frequency_penalty=config.frequency_penalty)
+            params = self._shared_params(B, dev, config)
         if histories is None and generated_tokens:
-            h = torch.tensor(list(generated_tokens), dtype=torch.int32)
-            histories = h.reshape(1, -1).expand(B, -1).to(dev)
-            history_lengths = torch.full((B,), h.numel(), dtype=torch.int32, device=dev)
+            histories, history_lengths = _upload_history(generated_tokens, B, dev)
         out = sample_rows(logits, params, uniforms, histories=histories, history_lengths=history_lengths,
                           logprobs=bool(config.logprobs), top_logprobs=int(config.top_logprobs),
                           generator=generator, allowed=allowed, row_kind_hint=hint)

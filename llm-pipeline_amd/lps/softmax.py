@@ -10,6 +10,7 @@ input dtype."""
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from typing import Optional, Tuple, Union
 
@@ -25,13 +26,18 @@ _WS = {}
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """Zero-filled scratch for split rows, cached per (device, stream): every
     launch leaves it zeroed, and launches on one stream never overlap."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, D.stream_of(device))
     with _WS_LOCK:
         t = _WS.get(key)
         if t is None or t.numel() < nbytes:
             t = torch.zeros((max(nbytes, 1 << 16),), dtype=torch.uint8, device=device)
             _WS[key] = t
         return t
+
+
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(rows: int, cols: int, dtype: int) -> int:
+    return _lib.load().lps_softmax_workspace_bytes(rows, cols, dtype)
 
 
 def fused_softmax(x: torch.Tensor, causal: bool = False, row_offset: int = 0,
@@ -79,8 +85,8 @@ def fused_softmax(x: torch.Tensor, causal: bool = False, row_offset: int = 0,
         a.stats_cols = stats_cols
     if rows:
         lib = _lib.load()
-        nb = lib.lps_softmax_workspace_bytes(rows, n_cols, a.dtype)
-        with torch.cuda.device(x.device):
+        nb = _workspace_bytes(rows, n_cols, a.dtype)
+        with D.guard(x.device):
             if nb:
                 ws = _workspace(x.device, nb)
                 a.workspace = ws.data_ptr()

@@ -12,6 +12,7 @@
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from dataclasses import dataclass
 from typing import Optional
@@ -29,13 +30,19 @@ def _spec_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """Zero-filled scratch for ``lps_spec_verify``, cached per (device,
     stream): every launch leaves it ready for the next, and launches on one
     stream never overlap."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, D.stream_of(device))
     with _WS_LOCK:
         t = _WS.get(key)
         if t is None or t.numel() < nbytes:
             t = torch.zeros((max(nbytes, 1 << 20),), dtype=torch.uint8, device=device)
             _WS[key] = t
         return t
+
+
+@functools.lru_cache(maxsize=256)
+def _spec_workspace_bytes(device_index: int, B: int, k: int, V: int) -> int:
+    """``lps_spec_workspace_bytes`` on the current device, a function of the sizes alone."""
+    return _lib.load().lps_spec_workspace_bytes(B, k, V)
 
 
 def verify_drafts_batched(target_probs: torch.Tensor, draft_probs: torch.Tensor, draft_tokens: torch.Tensor,
@@ -57,7 +64,7 @@ def verify_drafts_batched(target_probs: torch.Tensor, draft_probs: torch.Tensor,
     if q.numel() != K or t.numel() != K or u.numel() != K:
         raise ValueError("draft_probs, draft_tokens and rand_uniform must have K elements")
     out = torch.empty((K,), dtype=torch.int8, device=dev)
-    with torch.cuda.device(dev):
+    with D.guard(dev):
         rc = _lib.load().lps_verify_drafts(D.ptr(target_probs), dt, K, V, target_probs.stride(0),
                                            target_probs.stride(1), D.ptr(q), D.ptr(t), D.ptr(u), D.ptr(out),
                                            D.stream_of(dev))
@@ -105,11 +112,12 @@ def spec_verify(target_logits: torch.Tensor, draft_logits: torch.Tensor, draft_t
         draft_logits = draft_logits.contiguous()
     dev = target_logits.device
     dt = D.dtype_code(target_logits)
-    tok = draft_tokens.to(device=dev, dtype=torch.int64).reshape(B, k).contiguous()
-    ua = u_accept.to(device=dev, dtype=torch.float32).reshape(B, k).contiguous()
-    ur = u_resample.to(device=dev, dtype=torch.float32).reshape(B, k1).contiguous()
+    tok = D.on(draft_tokens, dev, torch.int64).reshape(B, k).contiguous()
+    ua = D.on(u_accept, dev, torch.float32).reshape(B, k).contiguous()
+    ur = D.on(u_resample, dev, torch.float32).reshape(B, k1).contiguous()
     lib = _lib.load()
-    ws_bytes = lib.lps_spec_workspace_bytes(B, k, V)
+    with D.guard(dev):
+        ws_bytes = _spec_workspace_bytes(dev.index, B, k, V)
     ws = _spec_workspace(dev, ws_bytes)
     out = SpecVerifyOutput(
         torch.empty((B,), dtype=torch.int32, device=dev),
@@ -144,7 +152,7 @@ def spec_verify(target_logits: torch.Tensor, draft_logits: torch.Tensor, draft_t
     a.row_status = D.ptr(out.status)
     a.workspace = D.ptr(ws)
     a.workspace_bytes = ws.numel()
-    with torch.cuda.device(dev):
+    with D.guard(dev):
         rc = lib.lps_spec_verify(ctypes.byref(a), D.stream_of(dev))
     _lib.check(rc, "lps_spec_verify")
     return out
