@@ -33,7 +33,9 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
   // (issued first so that they are not queued behind the chunk's 16-byte loads)
   RG_STAMP(0);
   const int32_t* hrow0 = P.history ? P.history + (int64_t)r * P.history_stride : nullptr;
-  const int hid = (hrow0 && (int64_t)tid < P.history_stride) ? hrow0[tid] : -1;
+  int hid = -1;
+  if (hrow0 && P.history_stride > 0) hid = (int64_t)tid < P.history_stride ? hrow0[tid] : -1;
+  else if (hrow0) hid = tid < g.hlen ? hrow0[tid] : -1;  // (a shared history is known to hold g.hlen ids only)
   CK C;
   C.load(row, v0, nv);
   C.mask(row_allowed(P, r), v0, nv);

@@ -77,3 +77,17 @@ def test_fast_small_and_ragged(dev):
             w = _small(V, 16, dt, seed=V)
             out = PY.run_workload(w, dev)
             PY.check_rows(w, out)
+
+
+@pytest.mark.parametrize("B", [3, 40])
+def test_one_history_shared_by_every_row(dev, B):
+    """A history of stride 0 (one row expanded to the batch) gives what its copies give."""
+    from lps import SamplingParams, sample_rows
+    g = torch.Generator().manual_seed(B)
+    x = torch.randn((B, 40000), generator=g).to(dev)
+    h = x[0].topk(300).indices.to(torch.int32).reshape(1, -1)         # the ids most likely to be drawn
+    p = SamplingParams.build(B, dev, top_k=50, repetition_penalty=1.5, frequency_penalty=2.0)
+    u = torch.rand((B,), generator=g).to(dev)
+    a = sample_rows(x, p, u, histories=h.expand(B, -1), logprobs=True)
+    b = sample_rows(x, p, u, histories=h.repeat(B, 1), logprobs=True)
+    assert torch.equal(a.tokens, b.tokens) and torch.equal(a.chosen_logprob, b.chosen_logprob)
