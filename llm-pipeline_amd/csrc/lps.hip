@@ -93,7 +93,9 @@ bool rg_wants_xf(const KParams& k, int flags) {
   const bool mt = !(flags & LPS_FLAG_ROWS_BASIC_FILTERS) &&
                   (k.min_p != nullptr || k.min_p_def > 0.0f || k.typical_p != nullptr || k.typical_p_def < 1.0f ||
                    k.top_k != nullptr || k.top_k_def > rg::FAST_KMAX);
-  return k.entropy || mt || ((k.skip_draw || (k.logits2 && k.skip_draw2)) && (k.top_p != nullptr || !(k.top_p_def < 1.0f)));
+  // (top-N logprobs of nucleus rows; greedy and top-k rows need none of it)
+  const bool tn = k.n_top > 0 && k.top_logprobs != nullptr && !(flags & LPS_FLAG_ROWS_TOPK);
+  return k.entropy || mt || tn || ((k.skip_draw || (k.logits2 && k.skip_draw2)) && (k.top_p != nullptr || !(k.top_p_def < 1.0f)));
 }
 
 // Launch shape of the row-group kernel for a batch: logits per thread (NE) of

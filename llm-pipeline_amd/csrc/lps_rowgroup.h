@@ -128,6 +128,8 @@ constexpr int FPT = CAPR / FT;     // finaliser: loaded entries per thread
 constexpr int FP1 = 4;             // finaliser: first-pass slots (loaded before the list lengths are known)
 constexpr int SEGCAP = 128;        // chunk: entries of one list per wave segment
 constexpr int CLMAX = NW * SEGCAP; // chunk: entries of one list
+constexpr int TLCAP = 128;         // chunk: top-N logprob entries of a nucleus row (64, and ties with the last)
+static_assert(CAPR / MAXG >= 2 * LPS_MAX_TOP_LOGPROBS, "a chunk's entries carry its top-N list, two words each");
 constexpr int LKM = CAPR;          // finaliser: loaded entries of one list (all chunks)
 constexpr int KM = 1024;           // finaliser: merged (sorted) entries of one list
 constexpr int KPT = KM / FT;       // merged entries per thread in the prefix scans
@@ -209,7 +211,9 @@ struct RgParams {
   float* fine;         // second-level bins: row r at fine + r * G * FHN (large top-k rows: one
                        // count byte per published bin instead)
   uint4* cands;        // row r at cands + r * CAPR: chunk j owns [j * capw, (j + 1) * capw): its
-                       // sorted list 1, then its sorted list 2, entries {z key, index, x bits, 0}
+                       // sorted list 1, then its sorted list 2, entries {z key, index, x bits, 0};
+                       // nucleus rows with top-N logprobs: the fourth words of its first 2 N
+                       // entries are its top-N list (index, x bits)
   int capw;            // list entries per chunk
 };
 
@@ -280,7 +284,7 @@ __device__ __forceinline__ RowCfg row_cfg(const KParams& P, int r) {
   else if (!MT) {
     if (g.minp > 0.0f || g.typp < 1.0f || g.ntop > 0) mode = MODE_DEFER;
     else mode = g.topp < 1.0f ? MODE_NUCLEUS : MODE_PURE;
-  } else if (g.ntop > 0 || g.minp > 1.0f) mode = MODE_DEFER;
+  } else if (g.minp > 1.0f) mode = MODE_DEFER;
   // (typical-p after a filter that removed ids keeps the argmax; on a full row
   // it is a threshold cut like min-p's)
   else mode = (g.topp < 1.0f || g.minp > 0.0f || g.typp < 1.0f) ? MODE_NUCLEUS : MODE_PURE;
@@ -388,6 +392,7 @@ struct RgChunkS : RgX {
     // lists fill): count << 48 | sum of low 8 mantissa bits
     unsigned long long fh[FHN];
   };
+  uint4 tl[TLCAP];  // nucleus rows with top-N logprobs: the chunk's largest logits, sorted
 };
 struct RgFinalS : RgX {
   uint64_t lk[2][LKM];                  // loaded lists, chunk by chunk (sorted within a chunk)
@@ -834,15 +839,20 @@ __device__ __forceinline__ void seg_done(RgLists& L, int l, uint32_t n) {
   if ((threadIdx.x & 63) == 0) L.scnt[l][threadIdx.x >> 6] = n > (uint32_t)SEGCAP ? SEGCAP + 1 : (int)n;
 }
 
+// Word i of a chunk's published top-N list: entry i / 2's index, then its logit.
+__device__ __forceinline__ uint32_t topn_word(const uint4* tl, int i) { return i & 1 ? tl[i >> 1].z : tl[i >> 1].y; }
+
 // Sorts the chunk's lists l < nl (their wave segments complete; the caller
 // barriers after seg_done) by key, descending, and writes them to dst: list 0
 // at [0, np0), list 1 at [np0, np0 + np1), entries {z key, index, x bits, 0}.  List 0
 // stops after rank lim0 - 1 and the entries whose z equals that entry's z
 // (lim0 = 0: no limit).  np[l] receives the counts; returns false when a
 // segment overflowed or the lists, list 0 after its limit, exceed cap
-// (nothing written then).  Every thread calls it; it ends with a barrier.
+// (nothing written then).  wl: the fourth words of the entries dst[0, nwl) carry
+// topn_word(wl, i) instead of 0 (entries past the lists: that word alone is
+// written).  Every thread calls it; it ends with a barrier.
 __device__ __forceinline__ bool sort_publish(RgLists& L, RgX& X, int nl, int lim0, bool greedy, float T, uint4* dst, int cap,
-                                             int (&np)[2]) {
+                                             int (&np)[2], const uint4* wl = nullptr, int nwl = 0) {
   const int tid = threadIdx.x;
   int n[2] = {0, 0}, pre[2][NW];
   bool over = false;
@@ -942,8 +952,11 @@ __device__ __forceinline__ bool sort_publish(RgLists& L, RgX& X, int nl, int lim
     const int f = l ? e - n[0] : e;
     if (l == 0 && rk[it] >= np0) continue;
     const uint64_t key = L.ck[l][f];
-    dst[(l ? np0 : 0) + rk[it]] = make_uint4(key_z(key), (uint32_t)key_index(key), L.cx[l][f], 0u);
+    const int at = (l ? np0 : 0) + rk[it];
+    dst[at] = make_uint4(key_z(key), (uint32_t)key_index(key), L.cx[l][f], wl && at < nwl ? topn_word(wl, at) : 0u);
   }
+  if (wl)
+    for (int i = np0 + n[1] + tid; i < nwl; i += NT) dst[i].w = topn_word(wl, i);
   np[0] = np0;
   np[1] = n[1];
   __syncthreads();

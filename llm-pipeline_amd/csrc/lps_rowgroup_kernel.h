@@ -67,6 +67,25 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     for (int i = 0; i < HB * 8 / 16 / NT; i++) h4[i * NT + tid] = u32x4{0u, 0u, 0u, 0u};
   }
   const float M = bred(tm, S.f, OpMax{});
+  // nucleus and pure rows with top-N logprobs: the chunk's N largest logits,
+  // sorted, kept in LDS until the candidates are published (the same
+  // threshold, segments and sort as a top-k row's; the counts, which the lists
+  // overlay, are used up)
+  const bool topn = XF && g.ntop > 0 && (mode == MODE_NUCLEUS || mode == MODE_PURE);
+  if (__builtin_expect(topn, 0)) {
+    const uint32_t v1[1] = {f2key(tm)};
+    uint32_t th = bred(wave_kth_largest<1>(v1, (uint32_t)((g.ntop + NW - 1) / NW)), S.u, OpMin{});
+    if (th > kNegInfKey + 1u && th != 0xFFFFFFFFu) th = f2key(collision_lo(key2f(th), T));
+    const float xth = fmaxf(key2f(th), -3.40282347e38f);
+    uint32_t n = 0;
+#pragma unroll
+    for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(v0, s));
+    seg_done(S.l, 0, n);
+    __syncthreads();
+    int np[2];
+    if (!sort_publish(S.l, S, 1, g.ntop, false, T, S.tl, TLCAP, np)) flags |= RF_OVERFLOW;
+    for (int i = np[0] + tid; i < g.ntop; i += NT) S.tl[i] = make_uint4(0u, 0xFFFFFFFFu, 0u, 0u);
+  }
   if (hist_mode) {  // the second level's bins (over the counts, read until that barrier)
     static_assert(FHN * 8 / 16 == NT, "one store per thread");
     reinterpret_cast<u32x4*>(S.fh)[tid] = u32x4{0u, 0u, 0u, 0u};
@@ -178,6 +197,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     sm.zsum = bred(zs, S.d, OpAdd{});
     sm.nanbin = bred(nanc, S.u, OpAdd{});
     if constexpr (XF) sm.zent = bred(zh, S.d3, OpAdd{});
+    if (topn)
+      for (int i = tid; i < 2 * g.ntop; i += NT) cbase[i].w = topn_word(S.tl, i);
   }
 
   if (hist_mode) {
@@ -821,7 +842,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     __syncthreads();
     RG_STAMP(13);
     int np[2];
-    if (!sort_publish(S.l, S, 2, 0, false, T, cbase, F.capw, np)) flags |= RF_OVERFLOW;
+    if (!sort_publish(S.l, S, 2, 0, false, T, cbase, F.capw, np, XF && topn ? S.tl : nullptr, 2 * g.ntop))
+      flags |= RF_OVERFLOW;
     sm.n1 = (uint16_t)np[0];
     sm.n2 = (uint16_t)np[1];
     sm.ab1 = 0.0; sm.ab2 = 0.0; sm.nab1 = 0;
@@ -1605,6 +1627,33 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
     }
   }
   if (row_skips_draw(P, r) && !greedy) token = -1;
+
+  if (XF && __builtin_expect(hmode && g.ntop > 0, 0)) {
+    // ---- top-N logprobs of a nucleus or pure row: the chunks' lists merged
+    // (at most 16 x 64 entries; the candidates are used up) ----
+    if (status) return 15;
+    const int nt = g.ntop;
+    __syncthreads();
+    for (int f = tid; f < G * nt; f += FT) {
+      const int cc = f / nt;
+      const uint4* e = cands + cc * capw + 2 * (f - cc * nt);
+      const uint32_t idx = ld_pub(&e[0].w), xb = ld_pub(&e[1].w);
+      S.lk[0][f] = idx == 0xFFFFFFFFu ? 0ull : cand_key(__uint_as_float(xb), (int)idx, false, T);
+      S.lx[0][f] = xb;
+    }
+    if (tid < G) {
+      S.cn[0][tid] = nt;
+      S.cb[0][tid] = tid * nt;
+      S.cn[1][tid] = S.cb[1][tid] = 0;
+    }
+    __syncthreads();
+    merge_lists_g(S, G, 32 - __builtin_clz((uint32_t)nt), G * nt, 0, Rm);
+    __syncthreads();
+    // (absent entries have key 0 and rank under every other; a row with fewer
+    // than N finite logits is left to the general kernel)
+    ntop_out = nt < V ? nt : V;
+    if (S.sk[0][ntop_out - 1] == 0ull) return 15;
+  }
 
   // ---- outputs ----
   // ln of sum exp(z) over the row: Z is in units of 2^Rref of exp2(x c)

@@ -79,6 +79,44 @@ def test_fast_small_and_ragged(dev):
             PY.check_rows(w, out)
 
 
+@pytest.mark.parametrize("B,V,dtype", [(3, 151936, torch.bfloat16), (64, 151936, torch.bfloat16), (20, 100001, torch.float16),
+                                       (5, 32001, torch.float32), (96, 40000, torch.float32)])
+@pytest.mark.parametrize("n_top", [1, 20, 64])
+def test_top_logprobs_of_nucleus_rows(dev, B, V, dtype, n_top):
+    """Top-N logprobs of rows without top-k (nucleus, min-p, typical-p, pure, and
+    a few greedy and top-k rows between them) on the row-group kernel, from one
+    chunk per row to 13 and on rows read element by element: every row on the
+    fast kernel, outputs against the oracle, ids exactly."""
+    w = W.c2(B=B, V=V, H=64)
+    i = torch.arange(B)
+    w.logits = w.logits.to(dtype)
+    w.temperature = torch.where(i % 7 == 6, torch.tensor(0.0), w.temperature.clamp(min=0.3))
+    w.top_k = torch.where(i % 5 == 4, torch.tensor(40), torch.tensor(0)).to(torch.int32)
+    w.top_p = torch.tensor([0.9, 1.0, 0.95, 0.5])[i % 4]
+    w.min_p = torch.where(i % 6 == 2, torch.tensor(0.05), torch.tensor(0.0))
+    w.logprobs, w.n_top = True, n_top
+    out = PY.run_workload(w, dev, row_kind_hint=0)
+    assert int(out.row_path.sum()) == 0
+    PY.check_rows(w, out, rows=range(0, B, 1 if B < 32 else 7), lp=True)
+
+
+def test_top_logprobs_left_to_the_general_kernel(dev):
+    """Rows with fewer legal ids than top_logprobs, and rows that cannot be
+    sampled, keep the general kernel's outputs."""
+    from lps import SamplingParams, sample_rows
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn((4, 5000), generator=g)
+    x[1, 10:] = float("-inf")
+    x[2, 7] = float("nan")
+    p = SamplingParams.build(4, dev, top_p=0.9)
+    u = torch.rand((4,), generator=g).to(dev)
+    a = sample_rows(x.to(dev), p, u, logprobs=True, top_logprobs=20)
+    b = sample_rows(x.to(dev), p, u, logprobs=True, top_logprobs=20, path="generic")
+    assert a.row_path.tolist() == [0, 1, 1, 0]
+    assert torch.equal(a.tokens, b.tokens) and torch.equal(a.status, b.status) and torch.equal(a.top_ids[:2], b.top_ids[:2])
+    torch.testing.assert_close(a.top_logprobs[[0, 1, 3]], b.top_logprobs[[0, 1, 3]], rtol=1e-5, atol=2e-6)
+
+
 @pytest.mark.parametrize("B", [3, 40])
 def test_one_history_shared_by_every_row(dev, B):
     """A history of stride 0 (one row expanded to the batch) gives what its copies give."""
