@@ -402,7 +402,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     // doubles, whose bit patterns order as they do
     if (tid == 0) {
       S.mi[0] = 1 << 30; S.mi[1] = -1; S.mi[2] = 1 << 30; S.mi[3] = -1;
-      S.u3[0] = 0u;
+      S.u3[0] = S.u3[1] = 0u;
       S.mq[0] = ~0ull;
       S.mq[1] = 0ull;
       S.mq[2] = ~0ull;
@@ -542,6 +542,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     int hi1 = nuc ? S.mi[1] : (1 << 30);
     uint64_t q1t = S.mq[0], q1b = S.mq[1];
     if (topp_on && hi1 < 0) flags |= RF_REGION;
+    bool thr1 = tc;  // region 1 covers a threshold cut's boundary (else top-p's alone)
     if (__builtin_expect(tc, 0)) {
       // the top-p cut entirely above [lom, hm]: top-p alone decides (every id
       // it keeps passes min-p); entirely under it (or no top-p): the threshold
@@ -552,6 +553,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       } else if (!(mt > Pm + eps) && hi1 >= 0) {
         lo1 = min(lo1, lom); hi1 = max(hi1, hm);
         q1t = min(q1t, S.mq[5]); q1b = max(q1b, S.mq[6]);
+      } else {
+        thr1 = false;
       }
     }
     if (XF && targ) lo1 = hi1 = 1 << 30;
@@ -561,7 +564,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     if (XF && targ) { t_lo = -1.0; t_hi = -2.0; }  // (no draw region)
     {
       int lo = 1 << 30, hi = -1;
-      uint32_t nest = 0;  // elements in either region (an upper estimate: bin mass / the bin's least mass)
+      uint32_t nest1 = 0, nest2 = 0;  // elements of the regions (upper estimates: bin mass / the bin's least mass)
       uint64_t a2 = ~0ull;  // cumulative mass at region 2's top
       double a = sx;
 #pragma unroll
@@ -573,9 +576,13 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
           hi = max(hi, b);
           a2 = min(a2, __builtin_bit_cast(uint64_t, a));
         }
-        if (in2 || (b >= lo1 && b <= hi1))
-          nest += (uint32_t)ceilf(__fmul_rn((float)mrg[i], ldexpf(1.0f, 134 - ((b >> 7) + HE0))) /
-                                  (float)(128 + (b & 127)));
+        const bool in1 = b >= lo1 && b <= hi1;
+        if (in2 || in1) {
+          const uint32_t n = (uint32_t)ceilf(__fmul_rn((float)mrg[i], ldexpf(1.0f, 134 - ((b >> 7) + HE0))) /
+                                             (float)(128 + (b & 127)));
+          nest1 += in1 ? n : 0u;
+          nest2 += in2 ? n : 0u;
+        }
         a += mrg[i];
       }
       if (hi >= 0) {
@@ -583,22 +590,31 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
         atomicMax(&S.mi[3], hi);
         atomicMin(reinterpret_cast<unsigned long long*>(&S.mq[2]), (unsigned long long)a2);
       }
-      if (nest) atomicAdd(&S.u3[0], nest);
+      if (nest1) atomicAdd(&S.u3[0], nest1);
+      if (nest2) atomicAdd(&S.u3[1], nest2);
     }
     __syncthreads();
     const int lo2 = S.mi[2];
     const int hi2 = S.mi[3];
-    const uint32_t nest = S.u3[0];
+    const uint32_t nest1 = S.u3[0], nest2 = S.u3[1];
     if (!(XF && targ) && (hi2 < 0 || !rfin)) flags |= RF_REGION;
     const bool need2 = !row_skips_draw(P, r);
     // ---- crowded regions take the second level (a row-uniform decision: every
     // chunk merged the same bins; a chunk whose first barrier timed out is
     // deferred, and counts itself at the second barrier without waiting) ----
     // (past 3/4 of the row's lists, so that no chunk's share passes its own
-    // list, or half of what the chunks' wave segments take)
-    const bool crowded = __builtin_expect(nest > (uint32_t)min(CAPR * 3 / 4, G * CLMAX / 2), 0);
-    const bool refine = crowded && !tc && !S.mi[6] && rfin && (!nuc || (hi1 >= 0 && hi1 - lo1 < RW)) &&
-                        (!need2 || (hi2 >= 0 && hi2 - lo2 < RW));
+    // list, or half of what the chunks' wave segments take, or more entries of
+    // one region than the finaliser merges)
+    const bool crowded = __builtin_expect(nest1 + nest2 > (uint32_t)min(CAPR * 3 / 4, G * CLMAX / 2) ||
+                                          nest1 > (uint32_t)KM || nest2 > (uint32_t)KM, 0);
+    // a threshold cut's region 1 stays whole bins (it has to cover the
+    // boundary's whole range) and must fit by itself: only the draw's is
+    // refined.  (Flat rows: min_p below every logit's ratio, the draw's bin
+    // holds thousands.)  Large top-k rows keep their counts in the fine bins' area
+    const bool fits1 = thr1 && !(XF && g.bigk) && nest1 <= (uint32_t)min(KM * 3 / 4, G * CLMAX / 4);
+    const bool fine1 = nuc && !thr1;   // region 1 is refined
+    const bool refine = crowded && (!thr1 || (fits1 && need2)) && !S.mi[6] && rfin &&
+                        (!fine1 || (hi1 >= 0 && hi1 - lo1 < RW)) && (!need2 || (hi2 >= 0 && hi2 - lo2 < RW));
     if (crowded && !refine) flags |= RF_WIDE;
     if (S.mi[6] && tid == 0) add_agent(ctr + CTR_FINE, 1u);
     // the regions in row bins (empty: 1 << 30), and in this chunk's bins
@@ -625,7 +641,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     uint32_t fnab = 0;
     if (__builtin_expect(refine, 0)) {
       // slot p of region q holds the fine bin F0 - p of its top bin (mass descending)
-      const int F0a = cr[1] < NOB ? (h1 + 1) * FSUB - 1 : -1, F0b = need2 ? (h2 + 1) * FSUB - 1 : -1;
+      const int F0a = fine1 && cr[1] < NOB ? (h1 + 1) * FSUB - 1 : -1, F0b = need2 ? (h2 + 1) * FSUB - 1 : -1;
       // (1) this chunk's fine bins of the region bins (the masses recomputed as binned)
 #pragma unroll
       for (int k = 0; k < NE / 2; k++) {
@@ -633,7 +649,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
         if (__builtin_amdgcn_ballot_w64((t1 | t2) != 0u) == 0ull) continue;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-          const bool o1 = (t1 >> (16 * h) & 0xFFFFu) != 0u, o2 = (t2 >> (16 * h) & 0xFFFFu) != 0u;
+          const bool o1 = fine1 && (t1 >> (16 * h) & 0xFFFFu) != 0u, o2 = (t2 >> (16 * h) & 0xFFFFu) != 0u;
           if (o1 || o2) {
             const float e = emass(C.x[2 * k + h], c, ref);
             const int f = efine(e);
@@ -700,7 +716,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       double a = inc - ms;
 #pragma unroll
       for (int i = 0; i < NW; i++) a += (i < wv && (i >= NW / 2) == q2) ? S.d3[i] : 0.0;
-      if (!q2 && nuc) {
+      if (!q2 && fine1) {
         a += __builtin_bit_cast(double, S.mq[0]);
         int lo = NOB, hi = -1;
         uint64_t at = ~0ull, ab = 0ull;
@@ -724,8 +740,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       __syncthreads();
       if (q2 && need2) {
         a += __builtin_bit_cast(double, S.mq[2]);
-        const double tl = (nuc ? (double)u * __builtin_bit_cast(double, S.mq[3]) : (double)u * Z) - eps;
-        const double th = (nuc ? (double)u * __builtin_bit_cast(double, S.mq[4]) : (double)u * Z) + eps;
+        const double tl = (nuc ? (double)u * __builtin_bit_cast(double, fine1 ? S.mq[3] : q1t) : (double)u * Z) - eps;
+        const double th = (nuc ? (double)u * __builtin_bit_cast(double, fine1 ? S.mq[4] : q1b) : (double)u * Z) + eps;
         int lo = NOB, hi = -1;
 #pragma unroll
         for (int i = 0; i < 2; i++) {
@@ -743,8 +759,10 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       __syncthreads();
       RG_STAMP(21);
       const int fp[4] = {S.mi[10], S.mi[11], S.mi[13], S.mi[15]};
-      if ((nuc && fp[1] < 0) || (need2 && fp[3] < 0)) flags |= RF_REGION;
-      if (nuc) {
+      if ((fine1 && fp[1] < 0) || (need2 && fp[3] < 0)) flags |= RF_REGION;
+      if (nuc && !fine1) {
+        cf[0] = l1 * FSUB; cf[1] = h1 * FSUB + FSUB - 1;
+      } else if (nuc) {
         cf[0] = F0a - fp[1]; cf[1] = F0a - fp[0];
         fr[0] = (cr[1] + 1) * FSUB - 1 - fp[1]; fr[1] = (cr[1] + 1) * FSUB - 1 - fp[0];
       }
@@ -757,7 +775,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 #pragma unroll
       for (int i = 0; i < 2; i++) {
         const int p = p0 + i;
-        if (!q2 && nuc && p < fp[0]) { fab1 += fine_mass(F0a - p, acc[i]); fnab += (uint32_t)(acc[i] >> 48); }
+        if (!q2 && fine1 && p < fp[0]) { fab1 += fine_mass(F0a - p, acc[i]); fnab += (uint32_t)(acc[i] >> 48); }
         if (q2 && need2 && p < fp[2]) fab2 += fine_mass(F0b - p, acc[i]);
       }
       // (5) the fine regions as ranges of logits [first key reaching the low

@@ -129,3 +129,25 @@ def test_one_history_shared_by_every_row(dev, B):
     a = sample_rows(x, p, u, histories=h.expand(B, -1), logprobs=True)
     b = sample_rows(x, p, u, histories=h.repeat(B, 1), logprobs=True)
     assert torch.equal(a.tokens, b.tokens) and torch.equal(a.chosen_logprob, b.chosen_logprob)
+
+
+@pytest.mark.parametrize("V,dtype", [(151936, torch.bfloat16), (100001, torch.float32), (50257, torch.float16)])
+def test_flat_threshold_rows_stay_on_the_row_group_kernel(dev, V, dtype):
+    """Almost uniform rows with min-p under every logit's ratio (alone, and after
+    a top-p that cuts first): the draw's bin, and the top-p cut's, hold
+    thousands of logits and take the second level.  At most one row in 16 off
+    the fast kernel; kept sets and draws against the oracle."""
+    B = 32
+    w = W.c2(B=B, V=V, H=16)
+    g = torch.Generator().manual_seed(V)
+    i = torch.arange(B)
+    w.logits = (torch.randn((B, V), generator=g) * 0.1).to(dtype)
+    w.top_k = torch.zeros(B, dtype=torch.int32)
+    w.temperature = 0.5 + 0.7 * torch.rand(B, generator=g)
+    w.min_p = torch.tensor([0.02, 0.05, 0.1, 0.0])[i % 4]
+    w.top_p = torch.tensor([1.0, 0.95])[(i // 4) % 2]
+    out = PY.run_workload(w, dev)
+    assert int(out.row_path.sum()) <= B // 16
+    min_p, w.min_p = w.min_p, torch.zeros(B)      # (min-p removes nothing here: the oracle's top-p band applies)
+    assert float(min_p.max()) < float(torch.exp(-(w.logits.float().amax(1) - w.logits.float().amin(1)) / w.temperature).min())
+    PY.check_rows(w, out)
