@@ -104,16 +104,17 @@ struct RgPlan {
   int vpe, ne, G, cv, nvec, capw;
   bool ok;
 };
+int rg_max_chunks(int R, int V);
 RgPlan rg_plan(int dtype, bool vec, int R, int V, bool lean = false) {
   RgPlan p{};
-  p.vpe = !vec ? 1 : (dtype == LPS_DTYPE_F32 ? 4 : 8);
-  p.nvec = V / p.vpe;
+  p.vpe = dtype == LPS_DTYPE_F32 ? 4 : 8;
+  // (rows that are not whole aligned vectors begin up to vpe - 1 logits into one)
+  p.nvec = vec ? V / p.vpe : (V + 2 * (p.vpe - 1)) / p.vpe;
   auto chunks = [&](int ne) { return (p.nvec + rg::NT * (ne / p.vpe) - 1) / (rg::NT * (ne / p.vpe)); };
   // rows of small batches (fp32: up to 16 rows, 16-bit: up to 12): 24
   // logits per thread, so a row spreads over more workgroups (latency; a
-  // 16-bit Qwen3 row: 13 chunks instead of 4); rows read element by element:
-  // 40; otherwise 80
-  p.ne = p.vpe == 1 ? 40 : ((R <= (p.vpe == 4 ? 16 : 12) && chunks(24) <= rg::MAXG) ? 24 : 80);
+  // 16-bit Qwen3 row: 13 chunks instead of 4); otherwise 80
+  p.ne = (R <= (p.vpe == 4 ? 16 : 12) && chunks(24) <= rg::MAXG) ? 24 : 80;
   // up to 32 rows: 40 per thread while every chunk still fits one resident
   // round (a Qwen3 row: 8 chunks instead of 4)
   if (p.ne == 80 && R <= 32 && (long)((R + 7) / 8 * 8) * chunks(40) <= (long)device_cus()) p.ne = 40;
@@ -121,24 +122,28 @@ RgPlan rg_plan(int dtype, bool vec, int R, int V, bool lean = false) {
   // build without the extra features: 100 (fp32) or 104 (16-bit) logits per
   // thread when that takes fewer chunks per row (fewer rounds, each a little
   // longer; the other build would spill registers at that size)
-  if (lean && p.ne == 80) {
+  if (lean && vec && p.ne == 80) {
     const int wide = p.vpe == 4 ? 100 : 104;
     if (chunks(wide) < chunks(80) && (long)((R + 7) / 8 * 8) * chunks(80) > (long)device_cus()) p.ne = wide;
   }
+  // (a misaligned row may need one chunk more than the workspace is sized for)
+  if (!vec && p.ne < 80 && chunks(p.ne) > rg_max_chunks(R, V)) p.ne = 80;
   p.G = chunks(p.ne);
-  p.ok = p.G >= 1 && p.G <= rg::MAXG && V >= 1;
+  p.ok = p.G >= 1 && p.G <= (vec ? rg::MAXG : rg_max_chunks(R, V)) && V >= 1;
   p.cv = p.ok ? (p.nvec + p.G - 1) / p.G : 1;
   p.capw = p.ok ? (rg::CAPR / p.G) / rg::NW * rg::NW : 0;
   return p;
 }
 // The most chunks any dtype's plan uses for (R, V): sizes the workspace.
 int rg_max_chunks(int R, int V) {
-  int g = 1;
-  for (int d = 0; d < 2; d++)
-    for (int v = 0; v < 2; v++) {
-      const RgPlan p = rg_plan(d == 0 ? LPS_DTYPE_F32 : LPS_DTYPE_BF16, v == 1, R, V);
-      if (p.ok && p.G > g) g = p.G;
-    }
+  // (at least one chunk per 512 x 40 logits, while the row fits MAXG of those:
+  // misaligned rows of large batches then fit with room to spare)
+  const int n40 = (V + rg::NT * 40 - 1) / (rg::NT * 40);
+  int g = n40 <= rg::MAXG ? n40 : 1;
+  for (const int dtype : {LPS_DTYPE_F32, LPS_DTYPE_BF16}) {
+    const RgPlan p = rg_plan(dtype, true, R, V);
+    if (p.ok && p.G > g) g = p.G;
+  }
   return g;
 }
 
@@ -166,7 +171,7 @@ RgWs rg_layout(void* base, int R, int V) {
   return w;
 }
 
-template <int DT, int VPE, int NE>
+template <int DT, int VPE, int NE, bool MA = false>
 hipError_t launch_rg(rg::RgParams F, int flags, hipStream_t s) {
   const unsigned grid = (unsigned)((F.k.R + 7) / 8 * 8 * F.G);
   // batches of more than one resident round of chunk workgroups: greedy and
@@ -180,27 +185,25 @@ hipError_t launch_rg(rg::RgParams F, int flags, hipStream_t s) {
   bool big = false;
   const unsigned cus = (unsigned)device_cus();
   const unsigned lim = (flags & LPS_FLAG_ROWS_TOPK) ? cus : cus * 8u;
-  if constexpr (VPE > 1) big = grid > lim && F.k.V <= rg::STREAM_VMAX;
+  if constexpr (!MA) big = grid > lim && F.k.V <= rg::STREAM_VMAX;   // (it reads whole aligned vectors)
   const bool run_stream = big && !(flags & LPS_FLAG_ROWS_NUCLEUS);
   const bool run_rg = !(run_stream && (flags & LPS_FLAG_ROWS_TOPK));
-  if constexpr (VPE > 1) {
-    if (run_stream) {
-      F.stream_only = run_rg ? 0 : 1;
-      if (F.k.allowed) hipLaunchKernelGGL((st::stream_kernel<DT, VPE, true>), dim3(F.k.R), dim3(st::SNT), 0, s, F);
-      else hipLaunchKernelGGL((st::stream_kernel<DT, VPE, false>), dim3(F.k.R), dim3(st::SNT), 0, s, F);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      F.skip_topk = 1;
-    }
+  if (run_stream) {
+    F.stream_only = run_rg ? 0 : 1;
+    if (F.k.allowed) hipLaunchKernelGGL((st::stream_kernel<DT, VPE, true>), dim3(F.k.R), dim3(st::SNT), 0, s, F);
+    else hipLaunchKernelGGL((st::stream_kernel<DT, VPE, false>), dim3(F.k.R), dim3(st::SNT), 0, s, F);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    F.skip_topk = 1;
   }
   if (run_rg) {
     // the build with the extra features when the launch may need them (the
     // plans of more than 80 logits per thread are made only for the other)
     if (rg_wants_xf(F.k, flags)) {
-      if constexpr (NE <= 80) hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, true>), dim3(grid), dim3(rg::NT), 0, s, F);
+      if constexpr (NE <= 80) hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, true, MA>), dim3(grid), dim3(rg::NT), 0, s, F);
       else return hipErrorInvalidValue;
     } else {
-      hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, false>), dim3(grid), dim3(rg::NT), 0, s, F);
+      hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, false, MA>), dim3(grid), dim3(rg::NT), 0, s, F);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -209,12 +212,17 @@ hipError_t launch_rg(rg::RgParams F, int flags, hipStream_t s) {
   // 1024-thread workgroup per row (the others return at once)
   KParams G = F.k;
   G.only_status = F.status;
-  return launch_gen<DT, VPE == 1 ? 1 : (DT == LPS_DTYPE_F32 ? 4 : 8)>(G, s);
+  return launch_gen<DT, MA ? 1 : VPE>(G, s);
 }
 
 template <int DT>
-hipError_t dispatch_rg_dt(const rg::RgParams& F, const RgPlan& p, int flags, hipStream_t s) {
-  if (p.vpe == 1) return launch_rg<DT, 1, 40>(F, flags, s);
+hipError_t dispatch_rg_dt(const rg::RgParams& F, const RgPlan& p, bool vec, int flags, hipStream_t s) {
+  constexpr int VPE = DT == LPS_DTYPE_F32 ? 4 : 8;
+  if (!vec) {
+    if (p.ne == 24) return launch_rg<DT, VPE, 24, true>(F, flags, s);
+    if (p.ne == 40) return launch_rg<DT, VPE, 40, true>(F, flags, s);
+    return launch_rg<DT, VPE, 80, true>(F, flags, s);
+  }
   if constexpr (DT == LPS_DTYPE_F32) {
     if (p.ne == 24) return launch_rg<DT, 4, 24>(F, flags, s);
     if (p.ne == 40) return launch_rg<DT, 4, 40>(F, flags, s);
@@ -297,9 +305,9 @@ hipError_t run_sample(const KParams& P, int dtype, bool vec, void* ws, size_t ws
   F.cands = w.cands;
   F.capw = p.capw;
   switch (dtype) {
-    case LPS_DTYPE_F32: return dispatch_rg_dt<LPS_DTYPE_F32>(F, p, flags, s);
-    case LPS_DTYPE_BF16: return dispatch_rg_dt<LPS_DTYPE_BF16>(F, p, flags, s);
-    default: return dispatch_rg_dt<LPS_DTYPE_F16>(F, p, flags, s);
+    case LPS_DTYPE_F32: return dispatch_rg_dt<LPS_DTYPE_F32>(F, p, vec, flags, s);
+    case LPS_DTYPE_BF16: return dispatch_rg_dt<LPS_DTYPE_BF16>(F, p, vec, flags, s);
+    default: return dispatch_rg_dt<LPS_DTYPE_F16>(F, p, vec, flags, s);
   }
 }
 

@@ -199,7 +199,7 @@ struct RgParams {
   // barrier (max, reference, mass), [MAXG, MAXG + G) at the chunk's end
   int G;               // chunks per row
   int cv;              // vectors per chunk (the last chunk may hold fewer)
-  int nvec;            // vectors per row
+  int nvec;            // vectors per row (the most any row needs: misaligned rows begin inside one)
   int heavy_first;     // dispatch rows without top-k first
   int skip_topk;       // the streaming kernel's rows (stream_takes) ran there: skip them
   int stream_only;     // the row-group kernel is not launched: the streaming kernel defers the others
@@ -653,65 +653,110 @@ __device__ __forceinline__ double typical_dmin(double Z, double AH, float R, flo
 }
 
 // ---------------------------------------------------------------------------
-// The chunk: NE logits per thread, as NV vectors of VPE logits (VPE = 1 for
-// rows read element by element).  Slot s = i * VPE + e of thread t is logit
-// (v0 + t + i * NT) * VPE + e of the row.
+// The chunk: NE logits per thread, as NV vectors of VPE logits: slot s = i * VPE
+// + e of thread t is logit (v0 + t + i * NT) * VPE + e of the row.  MA: rows
+// that are not whole aligned vectors (an odd vocabulary starts every row
+// elsewhere in its 16-byte line).  Vectors then count from the line that holds
+// the row's first logit, `mis` logits into it; slots before and after the row
+// are -inf.  A build of its own: with both in one, by a uniform branch or with
+// the clamps always on, aligned batches lost 2 % (c2 38.5 -> 39.3 us).
 // ---------------------------------------------------------------------------
-template <int DT, int VPE, int NE>
+template <int DT, int VPE, int NE, bool MA>
 struct Chk {
   static constexpr int NV = NE / VPE;
   static constexpr int ES = DT == LPS_DTYPE_F32 ? 4 : 2;
   static_assert(NE % VPE == 0, "whole vectors");
-  static_assert(VPE == 1 || VPE * ES == 16, "16-byte vectors");
+  static_assert(VPE * ES == 16, "16-byte vectors");
   float x[NE];
 
   // Issues every load before any use; vectors past the chunk end read the
-  // chunk's last vector and become -inf.
-  __device__ __forceinline__ void load(const char* row, int v0, int nv) {
+  // chunk's last vector (MA: a whole vector of the row) and become -inf.  line:
+  // the row's first 16-byte line.  MA: the row's first and last vector, when
+  // they hold logits of other rows (or none), are read logit by logit.
+  __device__ __forceinline__ void load(const char* line, int v0, int nv, int mis, int V) {
     const int t = threadIdx.x;
-    if constexpr (VPE == 1) {
-      float raw[NE];
-#pragma unroll
-      for (int i = 0; i < NE; i++) raw[i] = load1<DT>(row, (int64_t)v0 + min(t + i * NT, nv - 1));
-#pragma unroll
-      for (int i = 0; i < NE; i++) x[i] = (t + i * NT) < nv ? raw[i] : -INFINITY;
-    } else {
-      u32x4 raw[NV];
+    const int end = mis + V;
+    const int f0 = mis ? 1 : 0, f1 = end / VPE - 1;   // the row's whole vectors
+    const int lo = f0 - v0, hi = min(nv - 1, f1 - v0);
+    u32x4 raw[NV];
+    if constexpr (!MA) {
 #pragma unroll
       for (int i = 0; i < NV; i++)
         raw[i] = __builtin_nontemporal_load(
-            reinterpret_cast<const u32x4*>(row + (int64_t)(v0 + min(t + i * NT, nv - 1)) * 16));
+            reinterpret_cast<const u32x4*>(line + (int64_t)(v0 + min(t + i * NT, nv - 1)) * 16));
+    } else if (f1 >= f0) {
 #pragma unroll
-      for (int i = 0; i < NV; i++) {
-        const bool ok = (t + i * NT) < nv;
-        const uint32_t w[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
-        if constexpr (DT == LPS_DTYPE_F32) {
+      for (int i = 0; i < NV; i++)
+        raw[i] = __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4*>(line + (int64_t)(v0 + max(min(t + i * NT, hi), lo)) * 16));
+    } else {
 #pragma unroll
-          for (int e = 0; e < 4; e++) x[i * 4 + e] = ok ? __uint_as_float(w[e]) : -INFINITY;
-        } else {
+      for (int i = 0; i < NV; i++) raw[i] = u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
-          for (int e = 0; e < 8; e++) {
-            const uint32_t h = (w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-            const float f = DT == LPS_DTYPE_BF16 ? __uint_as_float(h << 16) : f16_to_f32(h);
-            x[i * 8 + e] = ok ? f : -INFINITY;
-          }
+    for (int i = 0; i < NV; i++) {
+      const bool ok = (t + i * NT) < nv;
+      const uint32_t w[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+      if constexpr (DT == LPS_DTYPE_F32) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[i * 4 + e] = ok ? __uint_as_float(w[e]) : -INFINITY;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const uint32_t h = (w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
+          const float f = DT == LPS_DTYPE_BF16 ? __uint_as_float(h << 16) : f16_to_f32(h);
+          x[i * 8 + e] = ok ? f : -INFINITY;
         }
       }
     }
+    if constexpr (MA) {
+      if (mis != 0 && v0 == 0) partial(line, 0, 0, mis, end);
+      const int vt = end / VPE;   // the last vector, when the row ends inside it
+      if (end % VPE != 0 && vt >= v0 && vt - v0 < nv) partial(line, vt, vt - v0, mis, end);
+    }
   }
-  // Vocabulary index of slot s.
-  __device__ static __forceinline__ int index(int v0, int s) {
-    return (v0 + (int)threadIdx.x + (s / VPE) * NT) * VPE + (s % VPE);
+  // Vector vec of the row (the chunk's q-th), logit by logit.
+  __device__ __forceinline__ void partial(const char* line, int vec, int q, int mis, int end) {
+    const int iv = q / NT;   // uniform
+    if ((int)threadIdx.x != q % NT) return;
+    float f[VPE];
+#pragma unroll
+    for (int e = 0; e < VPE; e++) {
+      const int el = vec * VPE + e;
+      f[e] = el >= mis && el < end ? load1<DT>(line, el) : -INFINITY;
+    }
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+      if (i == iv) {
+#pragma unroll
+        for (int e = 0; e < VPE; e++) x[i * VPE + e] = f[e];
+      }
   }
-  // Illegal ids to -inf from the row's legality bits (one byte per vector).
-  __device__ __forceinline__ void mask(const uint8_t* am, int v0, int nv) {
+  // Vocabulary index of slot s (e0 = v0 * VPE - mis; outside [0, V) only where
+  // the slot is -inf padding).
+  __device__ static __forceinline__ int index(int e0, int s) {
+    return e0 + ((int)threadIdx.x + (s / VPE) * NT) * VPE + (s % VPE);
+  }
+  // Illegal ids to -inf from the row's legality bits (nb bytes; one byte holds
+  // a vector's bits when the row is aligned, two when it is not).
+  __device__ __forceinline__ void mask(const uint8_t* am, int nb, int v0, int nv, int mis) {
     if (!am) return;
     const int t = threadIdx.x;
     uint32_t b[NV];
+    if constexpr (!MA) {
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-      const int id0 = (v0 + min(t + i * NT, nv - 1)) * VPE;
-      b[i] = (uint32_t)am[id0 >> 3] >> (id0 & 7);
+      for (int i = 0; i < NV; i++) {
+        const int id0 = (v0 + min(t + i * NT, nv - 1)) * VPE;
+        b[i] = (uint32_t)am[id0 >> 3] >> (id0 & 7);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; i++) {
+        const int id0 = (v0 + max(min(t + i * NT, nv - 1), 0)) * VPE - mis;   // from -mis
+        const int k = id0 >> 3;
+        const uint32_t b0 = k >= 0 ? (uint32_t)am[min(k, nb - 1)] : 0u;
+        b[i] = (b0 | (uint32_t)am[min(k + 1, nb - 1)] << 8) >> (id0 & 7);
+      }
     }
 #pragma unroll
     for (int i = 0; i < NV; i++)
@@ -758,7 +803,7 @@ __device__ __forceinline__ bool build_counts(RgChunkS<NE>& S, const int32_t* hro
   __syncthreads();
   bool sat = false;
   auto add = [&](int id) {
-    if (id >= lo && id < lo + n) {
+    if (id >= max(lo, 0) && id < lo + n) {   // (lo < 0: a misaligned row's first vector)
       const int l = id - lo;
       const int sh = 16 * (l & 1);
       const uint32_t old = atomicAdd(&S.a.hc[l >> 1], 1u << sh);
@@ -773,33 +818,31 @@ __device__ __forceinline__ bool build_counts(RgChunkS<NE>& S, const int32_t* hro
 }
 // Penalties of the counted ids, applied in place (a vector whose counts are
 // all zero costs one LDS read and a branch).
-template <int DT, int VPE, int NE>
-__device__ __forceinline__ void apply_counts(Chk<DT, VPE, NE>& C, const uint32_t* hc, int nv, float rep, float pres,
+template <int DT, int VPE, int NE, bool MA>
+__device__ __forceinline__ void apply_counts(Chk<DT, VPE, NE, MA>& C, const uint32_t* hc, int nv, float rep, float pres,
                                              float freq) {
-  constexpr int NV = Chk<DT, VPE, NE>::NV;
+  constexpr int NV = Chk<DT, VPE, NE, MA>::NV;
   const int t = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const int vl = t + i * NT;
     if (vl >= nv) continue;
     const int l0 = vl * VPE;  // chunk-local id of the vector's first logit
-    uint32_t cw[(VPE + 1) / 2];  // the vector's counts, two per word
+    uint32_t cw[VPE / 2];  // the vector's counts, two per word
     if constexpr (VPE == 8) {
       const uint4 q = *reinterpret_cast<const uint4*>(hc + (l0 >> 1));
       cw[0] = q.x; cw[1] = q.y; cw[2] = q.z; cw[3] = q.w;
-    } else if constexpr (VPE == 4) {
+    } else {
       const uint2 q = *reinterpret_cast<const uint2*>(hc + (l0 >> 1));
       cw[0] = q.x; cw[1] = q.y;
-    } else {
-      cw[0] = (hc[l0 >> 1] >> (16 * (l0 & 1))) & 0xFFFFu;
     }
     uint32_t any = 0;
 #pragma unroll
-    for (int q = 0; q < (VPE + 1) / 2; q++) any |= cw[q];
+    for (int q = 0; q < VPE / 2; q++) any |= cw[q];
     if (!any) continue;
 #pragma unroll
     for (int e = 0; e < VPE; e++) {
-      const uint32_t cnt = VPE == 1 ? cw[0] : (cw[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
+      const uint32_t cnt = (cw[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
       if (cnt) C.x[i * VPE + e] = penalize(C.x[i * VPE + e], (int)cnt, rep, pres, freq);
     }
   }

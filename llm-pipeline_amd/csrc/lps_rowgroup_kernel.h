@@ -16,16 +16,20 @@ __device__ __forceinline__ bool wait_count(uint32_t* p, uint32_t n) {
 // ===========================================================================
 // Chunk phase.  Returns the row's mode (MODE_DEFER: nothing published).
 // ===========================================================================
-template <int DT, int VPE, int NE, bool XF>
+template <int DT, int VPE, int NE, bool XF, bool MA>
 __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, const int r, const int j,
                                            const RowCfg& g, const uint32_t epoch, int& tcase) {
-  using CK = Chk<DT, VPE, NE>;
+  using CK = Chk<DT, VPE, NE, MA>;
   const KParams& P = F.k;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int G = F.G;
   const int v0 = j * F.cv;
-  const int nv = min(F.cv, F.nvec - v0);
   const char* row = row_ptr<DT>(P, r);
+  // vectors count from the row's first 16-byte line (Chk): the chunk holds nv
+  // of them (none, when a row needs one vector less than the launch's rows may)
+  const int mis = MA ? (int)(reinterpret_cast<uintptr_t>(row) & 15) / CK::ES : 0;
+  const int nv = MA ? max(min(F.cv, (mis + P.V + VPE - 1) / VPE - v0), 0) : min(F.cv, F.nvec - v0);
+  const int e0 = v0 * VPE - mis;  // the id of the chunk's first slot
   RgSum* sums = F.sums + (int64_t)r * 2 * MAXG;
   uint32_t* ctr = F.counters + (int64_t)r * 32;
 
@@ -37,8 +41,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
   if (hrow0 && P.history_stride > 0) hid = (int64_t)tid < P.history_stride ? hrow0[tid] : -1;
   else if (hrow0) hid = tid < g.hlen ? hrow0[tid] : -1;  // (a shared history is known to hold g.hlen ids only)
   CK C;
-  C.load(row, v0, nv);
-  C.mask(row_allowed(P, r), v0, nv);
+  C.load(row - mis * CK::ES, v0, nv, mis, P.V);
+  C.mask(row_allowed(P, r), (P.V + 31) / 32 * 4, v0, nv, mis);
   if (g.mode == MODE_DEFER) return MODE_DEFER;
   const int mode = g.mode;
   const bool greedy = g.greedy;
@@ -48,7 +52,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 
   // ---- penalties ----
   if (g.pen) {
-    if (!build_counts<NE>(S, g.hrow, g.hlen, tid < g.hlen ? hid : -1, v0 * VPE, nv * VPE)) flags |= RF_HISTORY;
+    if (!build_counts<NE>(S, g.hrow, g.hlen, tid < g.hlen ? hid : -1, e0, nv * VPE)) flags |= RF_HISTORY;
     apply_counts(C, S.a.hc, nv, g.rep, g.pres, g.freq);
   }
 
@@ -67,19 +71,27 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     for (int i = 0; i < HB * 8 / 16 / NT; i++) h4[i * NT + tid] = u32x4{0u, 0u, 0u, 0u};
   }
   const float M = bred(tm, S.f, OpMax{});
+  // the m-th largest thread maximum of each wave that holds vectors (a short
+  // row fills the first ones only), m = ceil(k / waves): at least k logits of
+  // the chunk reach the least of them
+  auto kth_bound = [&](int k) -> uint32_t {
+    const int nw = MA ? max(min(NW, (nv + 63) >> 6), 1) : NW;
+    const uint32_t v1[1] = {f2key(tm)};
+    const uint32_t wth = wave_kth_largest<1>(v1, (uint32_t)((k + nw - 1) / nw));
+    return bred(!MA || wv < nw ? wth : 0xFFFFFFFFu, S.u, OpMin{});
+  };
   // nucleus and pure rows with top-N logprobs: the chunk's N largest logits,
   // sorted, kept in LDS until the candidates are published (the same
   // threshold, segments and sort as a top-k row's; the counts, which the lists
   // overlay, are used up)
   const bool topn = XF && g.ntop > 0 && (mode == MODE_NUCLEUS || mode == MODE_PURE);
   if (__builtin_expect(topn, 0)) {
-    const uint32_t v1[1] = {f2key(tm)};
-    uint32_t th = bred(wave_kth_largest<1>(v1, (uint32_t)((g.ntop + NW - 1) / NW)), S.u, OpMin{});
+    uint32_t th = kth_bound(g.ntop);
     if (th > kNegInfKey + 1u && th != 0xFFFFFFFFu) th = f2key(collision_lo(key2f(th), T));
     const float xth = fmaxf(key2f(th), -3.40282347e38f);
     uint32_t n = 0;
 #pragma unroll
-    for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(v0, s));
+    for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(e0, s));
     seg_done(S.l, 0, n);
     __syncthreads();
     int np[2];
@@ -114,7 +126,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     if (tn) {
 #pragma unroll
       for (int s = 0; s < NE; s++)
-        if (C.x[s] != C.x[s]) best = min(best, CK::index(v0, s));
+        if (C.x[s] != C.x[s]) best = min(best, CK::index(e0, s));
     }
     const int bnan = bred(best, S.i1, OpMin{});
     __syncthreads();
@@ -126,9 +138,11 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       if (tm == M) {
 #pragma unroll
         for (int s = 0; s < NE; s++)
-          if (C.x[s] == M) best = min(best, CK::index(v0, s));
+          if (C.x[s] == M) best = min(best, CK::index(e0, s));
       }
+      // (MA, all -inf: the first id, also where padding precedes it)
       sm.amax = bred(best, S.i2, OpMin{});
+      if (MA) sm.amax = max(sm.amax, 0);
     }
   }
 
@@ -149,17 +163,14 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     RG_STAMP(3);
     if (g.kprime > 0) {
       // ---- candidates: every logit at or above the chunk threshold ----
-      const uint32_t m = (uint32_t)((g.kprime + NW - 1) / NW);
-      const uint32_t v1[1] = {f2key(tm)};
-      const uint32_t wth = wave_kth_largest<1>(v1, m);
-      uint32_t th = bred(wth, S.u, OpMin{});
+      uint32_t th = kth_bound(g.kprime);
       RG_STAMP(12);
       if (!greedy && th > kNegInfKey + 1u && th != 0xFFFFFFFFu) th = f2key(collision_lo(key2f(th), T));
       // -inf is never a candidate (it has no mass); NaN always is (!(x < t))
       const float xth = fmaxf(key2f(th), -3.40282347e38f);
       uint32_t n = 0;
 #pragma unroll
-      for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(v0, s));
+      for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(e0, s));
       seg_done(S.l, 0, n);
       __syncthreads();
       RG_STAMP(13);
@@ -290,7 +301,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       if (tm >= xlo) {
 #pragma unroll
         for (int s = 0; s < NE; s++)
-          if (C.x[s] >= xlo) best = min(best, CK::index(v0, s));
+          if (C.x[s] >= xlo) best = min(best, CK::index(e0, s));
       }
       sm.amax = bred(best, S.i1, OpMin{});
     }
@@ -304,14 +315,17 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
         float mq = INFINITY;
 #pragma unroll
         for (int e = 0; e < VPE; e++) {
-          nq += C.x[q * VPE + e] == -INFINITY ? 1u : 0u;
-          mq = fminf(mq, C.x[q * VPE + e]);
+          const bool inf = C.x[q * VPE + e] == -INFINITY;
+          nq += inf ? 1u : 0u;
+          mq = inf ? mq : fminf(mq, C.x[q * VPE + e]);   // (used for rows without -inf)
         }
         const bool inr = tid + q * NT < nv;  // (vector q of this thread)
         ni += inr ? nq : 0u;
         mn = inr ? fminf(mn, mq) : mn;
       }
-      const uint32_t nis = bred(ni, S.u2, OpAdd{});
+      // (without the padding of the row's first and last vector)
+      const int pads = MA && nv > 0 ? max(-e0, 0) + max(e0 + nv * VPE - P.V, 0) : 0;
+      const uint32_t nis = bred(ni, S.u2, OpAdd{}) - (uint32_t)pads;
       sm.ab1 = tw_pack(nis, f2key(bred(mn, S.f, OpMin{})));
     }
     // ---- publish the summary and the bins, one barrier among the row's chunks ----
@@ -486,7 +500,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 #pragma unroll
         for (int s = 0; s < NE; s++) {
           const bool inr = tid + (s / VPE) * NT < nv;
-          nd += inr && C.x[s] < xt ? 1u : 0u;
+          nd += inr && C.x[s] < xt && C.x[s] != -INFINITY ? 1u : 0u;   // (such a row holds no -inf: padding)
           mk = inr && C.x[s] >= xt ? fminf(mk, C.x[s]) : mk;
         }
         const uint32_t nds = bred(nd, S.u2, OpAdd{});
@@ -838,8 +852,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const int s2 = 2 * k + h;
-          seg_put(S.l, 0, o[h][0], n1, C.x[s2], CK::index(v0, s2));
-          seg_put(S.l, 1, o[h][1], n2, C.x[s2], CK::index(v0, s2));
+          seg_put(S.l, 0, o[h][0], n1, C.x[s2], CK::index(e0, s2));
+          seg_put(S.l, 1, o[h][1], n2, C.x[s2], CK::index(e0, s2));
         }
       }
     } else {
@@ -850,8 +864,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const int s2 = 2 * k + h;
-          seg_put(S.l, 0, (t1 >> (16 * h) & 0xFFFFu) != 0u, n1, C.x[s2], CK::index(v0, s2));
-          seg_put(S.l, 1, (t2 >> (16 * h) & 0xFFFFu) != 0u, n2, C.x[s2], CK::index(v0, s2));
+          seg_put(S.l, 0, (t1 >> (16 * h) & 0xFFFFu) != 0u, n1, C.x[s2], CK::index(e0, s2));
+          seg_put(S.l, 1, (t2 >> (16 * h) & 0xFFFFu) != 0u, n2, C.x[s2], CK::index(e0, s2));
         }
       }
     }
@@ -1622,9 +1636,12 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
     if (!nuc && !(XF && tall) && P.kept_count) {
       // every finite logit is kept: count the -inf ones (a pass over the row)
       uint32_t ninf = 0;
-      const int nvec = F.nvec;
+      const bool al = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
+      const int nvec = al ? V / VPE : 0;
+      for (int i = nvec * VPE + tid; i < V; i += FT)   // a misaligned row, or the end of an odd one
+        ninf += (load1<DT>(row, i) == -INFINITY || !id_allowed(row_allowed(P, r), i)) ? 1u : 0u;
       for (int v = tid; v < nvec; v += FT) {
-        float xx[VPE > 1 ? VPE : 1];
+        float xx[VPE];
         loadv<DT, VPE>(row, (int64_t)v * VPE, xx);
         const uint8_t* am = row_allowed(P, r);
 #pragma unroll
@@ -1734,7 +1751,7 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
 // draw (the mass-only path), or may hold min-p / typical-p rows without top-k
 // or rows with top_k past FAST_KMAX; that code is absent otherwise (such rows
 // are then deferred).
-template <int DT, int VPE, int NE, bool XF>
+template <int DT, int VPE, int NE, bool XF, bool MA>
 __global__ __launch_bounds__(NT) void rowgroup_kernel(RgParams F) {
   __shared__ RgShared<NE> SU;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -1749,7 +1766,7 @@ __global__ __launch_bounds__(NT) void rowgroup_kernel(RgParams F) {
   // before any of them arrives
   const uint32_t epoch = ld_agent(F.counters + (int64_t)r * 32 + CTR_EPOCH);
   int tcase = -1;  // typical-p rows without other filters: TYP_*
-  const int mode = chunk_phase<DT, VPE, NE, XF>(F, SU.c, r, j, g, epoch, tcase);
+  const int mode = chunk_phase<DT, VPE, NE, XF, MA>(F, SU.c, r, j, g, epoch, tcase);
   if (mode == MODE_DEFER) {
     if (j == 0 && threadIdx.x == 0) F.status[r] = LPS_ROW_DEFERRED | (1 << 8);
     return;

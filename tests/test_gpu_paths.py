@@ -151,3 +151,38 @@ def test_flat_threshold_rows_stay_on_the_row_group_kernel(dev, V, dtype):
     min_p, w.min_p = w.min_p, torch.zeros(B)      # (min-p removes nothing here: the oracle's top-p band applies)
     assert float(min_p.max()) < float(torch.exp(-(w.logits.float().amax(1) - w.logits.float().amin(1)) / w.temperature).min())
     PY.check_rows(w, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,V", [(5, 9), (3, 1001), (3, 12289), (24, 50257), (2, 151935), (40, 100001), (70, 40963)])
+def test_rows_off_the_16_byte_lines(dev, dtype, B, V):
+    """Odd vocabularies (every row starts elsewhere in its 16-byte line, ids shift
+    by that much in the vectors) in every row mode, with histories and legality
+    masks, from a row of one partial vector to several chunks; the logits also
+    as rows of a wider buffer.  Rows against the oracle, none deferred for V
+    past the smallest."""
+    w = W.c2(B=B, V=V, H=64)
+    i = torch.arange(B)
+    g = torch.Generator().manual_seed(V)
+    legal = torch.rand((B, V), generator=g) < 0.7
+    legal[:, V // 2] = True
+    w.logits = w.logits.to(dtype).masked_fill(~legal, float("-inf"))   # (the oracle's rows)
+    raw = w.logits.masked_fill(~legal, 3.0).to(dev)
+    w.temperature = torch.where(i % 5 == 3, torch.tensor(0.0), w.temperature.clamp(min=0.3))
+    w.top_k = torch.where(i % 3 == 0, torch.tensor(0), w.top_k.clamp(max=V)).to(torch.int32)
+    w.min_p = torch.where(i % 6 == 3, torch.tensor(0.05), torch.tensor(0.0))
+    w.logprobs = True
+    out = PY.run_workload(w, dev, row_kind_hint=0)
+    PY.check_rows(w, out, rows=range(0, B, 1 if B < 30 else 7), lp=True)
+    assert int(out.row_path.sum()) == 0 or V < 2000
+    ref = out
+    w.logits = raw.cpu()
+    out = PY.run_workload(w, dev, row_kind_hint=0, allowed=legal.to(dev))
+    assert torch.equal(out.tokens, ref.tokens) and torch.equal(out.kept_count, ref.kept_count)
+    wide = torch.full((B, V + 5), 50.0, dtype=dtype, device=dev)       # rows from the fourth element on
+    wide[:, 3:3 + V] = raw
+    from lps import SamplingParams, sample_rows
+    p = SamplingParams(*[t.to(dev) for t in (w.temperature, w.top_k, w.top_p, w.min_p, w.typical_p, w.rep, w.pres, w.freq)])
+    o = sample_rows(wide[:, 3:3 + V], p, w.uniforms.to(dev), histories=w.histories.to(dev),
+                    history_lengths=w.hist_len.to(dev), allowed=legal.to(dev))
+    assert torch.equal(o.tokens, ref.tokens)
