@@ -59,9 +59,10 @@ def _upload_history(ids: List[int], B: int, dev: torch.device) -> tuple:
     the device, in one copy (from pinned memory, which does not wait for the
     stream, unless a graph is being captured)."""
     try:
-        h = torch.frombuffer(array("i", ids), dtype=torch.int32)
+        # (an array of bytes would take their memory, not their values)
+        h = torch.frombuffer(array("i", ids if isinstance(ids, list) else list(ids)), dtype=torch.int32)
     except (TypeError, OverflowError):   # (what torch converts or rejects)
-        h = torch.tensor(list(ids), dtype=torch.int32)
+        h = torch.tensor(list(ids), dtype=torch.int32).reshape(-1)
     n = h.numel()
     pin = not torch.cuda.is_current_stream_capturing()
     buf = torch.empty((n + B,), dtype=torch.int32, pin_memory=pin)
@@ -79,7 +80,6 @@ class Sampler:
     def __init__(self, config: Optional[SamplingConfig] = None):
         self.config = config or SamplingConfig()
         self.last_output = None
-        self._params = {}
 
     def _shared_params(self, B: int, dev: torch.device, config: "SamplingConfig") -> SamplingParams:
         """The config's values for every row as device tensors: 8 fills a call
@@ -93,11 +93,13 @@ class Sampler:
                 torch.cuda.is_current_stream_capturing():
             return SamplingParams.build(B, dev, *values)
         key = (B, dev.index, D.stream_of(dev), values)
-        p = self._params.get(key)
+        # (a subclass with its own __init__, or an older pickle, has none yet)
+        kept = self.__dict__.setdefault("_params", {})
+        p = kept.get(key)
         if p is None:
-            if len(self._params) >= self._PARAM_SETS:
-                self._params.clear()
-            p = self._params[key] = SamplingParams.build(B, dev, *values)
+            if len(kept) >= self._PARAM_SETS:
+                kept.clear()
+            p = kept[key] = SamplingParams.build(B, dev, *values)
         return p
 
     def sample_token(self, logits: torch.Tensor, config_override: Optional[Dict[str, Any]] = None,

@@ -186,3 +186,23 @@ def test_rows_off_the_16_byte_lines(dev, dtype, B, V):
     o = sample_rows(wide[:, 3:3 + V], p, w.uniforms.to(dev), histories=w.histories.to(dev),
                     history_lengths=w.hist_len.to(dev), allowed=legal.to(dev))
     assert torch.equal(o.tokens, ref.tokens)
+
+
+def test_single_request_call_takes_every_form_of_history(dev):
+    """A history as a list, a tuple, bytes, nested lists or whole floats is the
+    same history, also for a sampler whose class has an ``__init__`` of its own."""
+    from lps import Sampler, SamplingConfig
+
+    class Own(Sampler):
+        def __init__(self, config):
+            self.config = config
+
+    logits = torch.randn((1, 4099), generator=torch.Generator().manual_seed(7)).to(dev)
+    ids = [3, 250, 17, 3]
+    config = SamplingConfig(temperature=0.9, top_p=0.95, repetition_penalty=3.0, frequency_penalty=0.5, logprobs=True)
+    seen = []
+    for s in (Sampler(config), Own(config)):
+        for h in (ids, tuple(ids), bytes(ids), [ids], [float(i) for i in ids]):
+            t = s.sample_token(logits, generated_tokens=h, uniforms=torch.tensor([0.4], device=dev))
+            seen.append((torch.as_tensor(t).reshape(-1).tolist(), s.last_output.chosen_logprob.tolist()))
+    assert all(x == seen[0] for x in seen)
