@@ -18,7 +18,7 @@ from __future__ import annotations
 import math
 from array import array
 from dataclasses import dataclass
-from typing import Any, Dict, List, Optional
+from typing import Any, Dict, Iterable, List, Optional
 
 import torch
 
@@ -54,16 +54,26 @@ _CONFIG_KEYS = (
 )
 
 
-def _upload_history(ids: List[int], B: int, dev: torch.device) -> tuple:
-    """One history for every row: ``int32 [B, n]`` and lengths ``int32 [B]`` on
-    the device, in one copy (from pinned memory, which does not wait for the
-    stream, unless a graph is being captured)."""
+def _history_ids(tokens) -> torch.Tensor:
+    """A request's generated ids (any iterable, read once) as ``int32 [n]`` on the host."""
+    ids = list(tokens)
+    if not ids:
+        return torch.empty((0,), dtype=torch.int32)
     try:
         # (an array of bytes would take their memory, not their values)
-        h = torch.frombuffer(array("i", ids if isinstance(ids, list) else list(ids)), dtype=torch.int32)
+        return torch.frombuffer(array("i", ids), dtype=torch.int32)
     except (TypeError, OverflowError):   # (what torch converts or rejects)
-        h = torch.tensor(list(ids), dtype=torch.int32).reshape(-1)
+        return torch.tensor(ids, dtype=torch.int32).reshape(-1)
+
+
+def _upload_history(tokens: Iterable[int], B: int, dev: torch.device) -> tuple:
+    """One history for every row: ``int32 [B, n]`` and lengths ``int32 [B]`` on
+    the device, in one copy (from pinned memory, which does not wait for the
+    stream, unless a graph is being captured); ``(None, None)`` without ids."""
+    h = _history_ids(tokens)
     n = h.numel()
+    if n == 0:
+        return None, None
     pin = not torch.cuda.is_current_stream_capturing()
     buf = torch.empty((n + B,), dtype=torch.int32, pin_memory=pin)
     buf[:n] = h

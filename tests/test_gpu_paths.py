@@ -206,3 +206,22 @@ def test_single_request_call_takes_every_form_of_history(dev):
             t = s.sample_token(logits, generated_tokens=h, uniforms=torch.tensor([0.4], device=dev))
             seen.append((torch.as_tensor(t).reshape(-1).tolist(), s.last_output.chosen_logprob.tolist()))
     assert all(x == seen[0] for x in seen)
+
+
+def test_single_request_call_reads_iterators_once(dev):
+    """A history that can be read only once, of ids or of floats, is the
+    list's history; an empty iterator is no history."""
+    from lps import Sampler, SamplingConfig
+    logits = torch.randn((2, 4099), generator=torch.Generator().manual_seed(8)).to(dev)
+    u = torch.tensor([0.4, 0.7], device=dev)
+    s = Sampler(SamplingConfig(temperature=0.9, top_p=0.95, repetition_penalty=3.0, frequency_penalty=0.5, logprobs=True))
+
+    def call(h):
+        t = s.sample_token(logits, generated_tokens=h, uniforms=u)
+        return t.tolist(), s.last_output.chosen_logprob.tolist()
+
+    ids = logits[0].topk(40).indices.tolist()
+    want = call(ids)
+    assert want != call(None)
+    assert call(iter(ids)) == want and call(float(i) for i in ids) == want
+    assert call(iter([])) == call(None)
