@@ -82,6 +82,15 @@ def _upload_history(tokens: Iterable[int], B: int, dev: torch.device) -> tuple:
     return buf[:n].unsqueeze(0).expand(B, n).contiguous(), buf[n:]
 
 
+class _KeptParams(dict):
+    """Parameter sets kept by a sampler.  A deep copy or a pickle of the sampler
+    starts with none: copied tensors would be filled on the stream of the copy,
+    not on the one that their key names."""
+
+    def __reduce__(self):
+        return _KeptParams, ()
+
+
 class Sampler:
     """Centralised logits -> token sampler on MI355X."""
 
@@ -104,7 +113,7 @@ class Sampler:
             return SamplingParams.build(B, dev, *values)
         key = (B, dev.index, D.stream_of(dev), values)
         # (a subclass with its own __init__, or an older pickle, has none yet)
-        kept = self.__dict__.setdefault("_params", {})
+        kept = self.__dict__.setdefault("_params", _KeptParams())
         p = kept.get(key)
         if p is None:
             if len(kept) >= self._PARAM_SETS:

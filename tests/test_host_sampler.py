@@ -1,9 +1,13 @@
 """The host side of a single-request call (CPU, no GPU)."""
 
+import copy
+import pickle
+
 import numpy as np
 import pytest
 import torch
 
+from lps import Sampler, SamplingConfig
 from lps.sampling import _history_ids, _upload_history
 
 
@@ -43,3 +47,20 @@ def test_generated_tokens_rejected(bad):
 
 def test_empty_iterators_are_no_history():
     assert _upload_history(iter([]), 2, torch.device("cpu")) == (None, None)
+
+
+@pytest.mark.parametrize("duplicate", [copy.deepcopy, lambda s: pickle.loads(pickle.dumps(s))])
+def test_copies_of_a_sampler_keep_no_parameter_tensors(monkeypatch, duplicate):
+    """The kept parameter sets belong to the stream that filled them: a copy,
+    whose tensors another stream would have filled, makes its own."""
+    import lps.sampling as S
+    monkeypatch.setattr(S.D, "stream_of", lambda dev: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    s = Sampler(SamplingConfig(temperature=0.7))
+    dev = torch.device("cpu")
+    kept = s._shared_params(2, dev, s.config)
+    assert s._shared_params(2, dev, s.config) is kept
+    d = duplicate(s)
+    assert d.config == s.config and not d._params
+    assert d._shared_params(2, dev, d.config) is not kept
+    assert s._shared_params(2, dev, s.config) is kept
