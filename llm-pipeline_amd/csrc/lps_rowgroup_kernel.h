@@ -52,7 +52,9 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 
   // ---- penalties ----
   if (g.pen) {
-    if (!build_counts<NE>(S, g.hrow, g.hlen, tid < g.hlen ? hid : -1, e0, nv * VPE)) flags |= RF_HISTORY;
+    // (a misaligned row may end inside its last vector: ids from V on count nowhere)
+    const int nids = MA ? min(nv * VPE, P.V - e0) : nv * VPE;
+    if (!build_counts<NE>(S, g.hrow, g.hlen, tid < g.hlen ? hid : -1, e0, nids)) flags |= RF_HISTORY;
     apply_counts(C, S.a.hc, nv, g.rep, g.pres, g.freq);
   }
 

@@ -380,3 +380,25 @@ def test_top_k_past_the_lists(run_case, tmp_path, dtype, V):
     print("rows off the row-group kernel:", off, out.reasons)
     assert len(off) <= B // 4, (off, out.reasons)
     PY.check_rows(w, out)
+
+
+@pytest.mark.parametrize("V,dtype", [(4099, torch.bfloat16), (4093, torch.float32)])
+def test_history_ids_past_an_odd_vocabulary(run_case, tmp_path, dtype, V):
+    """History ids in [V, V + 7) count nowhere, also where a misaligned row's
+    last vector has slots for them: with a repetition penalty of 0 (-inf * 0 is
+    NaN) and with 65534 repeats of V (a count that would saturate) the rows
+    are sampled on the row-group kernel as without a history."""
+    B, n = 4, 65600
+    w = _small(V, B, dtype, seed=V)
+    w.temperature, w.top_k = torch.full((B,), 0.9), torch.tensor([0, 20] * (B // 2), dtype=torch.int32)
+    w.top_p, w.min_p, w.typical_p = torch.full((B,), 0.9), torch.zeros(B), torch.ones(B)
+    w.rep, w.pres, w.freq = torch.zeros(B), torch.zeros(B), torch.zeros(B)
+    w.histories, w.hist_len = None, None
+    want = _run(run_case, w, tmp_path)
+    w.histories = torch.full((B, n), V, dtype=torch.int32)
+    w.histories[:, :14] = torch.cat([V + torch.arange(7), -1 - torch.arange(7)]).to(torch.int32)
+    w.hist_len = torch.full((B,), n, dtype=torch.int32)
+    got = _run(run_case, w, tmp_path)
+    assert (got.row_path == 0).all() and (want.row_path == 0).all(), (got.reasons, want.reasons)
+    assert torch.equal(got.tokens, want.tokens) and torch.equal(got.status, want.status)
+    assert torch.equal(got.kept_count, want.kept_count) and torch.equal(got.kept_cut, want.kept_cut)
