@@ -932,6 +932,7 @@ int lps_softmax(const lps_softmax_args* a, void* stream) {
       }
     } else {
       S.G = 1;
+      S.records = a->out;   // (unused: a non-null base for the address that the kernel forms)
     }
     if (p.kind != 2) {
       switch (a->dtype) {

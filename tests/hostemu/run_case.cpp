@@ -5,11 +5,14 @@
 //
 //   run_case IN OUT
 //
-// IN holds one lps_sample call's inputs, OUT receives its outputs (layouts
-// below, little-endian).  The workspace is calloc'd at its exact size, so an
+// IN holds one call's inputs, OUT receives its outputs (layouts below,
+// little-endian); the first word says which entry point: lps_sample,
+// lps_lm_head, lps_softmax or lps_spec_verify.  The workspace is calloc'd at its exact size, so an
 // access past it, past any input or output array, or past an LDS array of a
 // kernel, stops the run with the sanitizer's report.
 #include "../../llm-pipeline_amd/csrc/lps.hip"
+
+#include <sanitizer/asan_interface.h>
 
 #include <vector>
 
@@ -40,6 +43,160 @@ void wr(FILE* f, const std::vector<T>& v) {
   if (!v.empty()) fwrite(v.data(), sizeof(T), v.size(), f);
 }
 
+// A heap copy of exactly the array's size.
+template <typename T>
+T* exact(const std::vector<T>& v) {
+  T* p = static_cast<T*>(malloc(v.size() * sizeof(T)));
+  if (!v.empty()) memcpy(p, v.data(), v.size() * sizeof(T));
+  return p;
+}
+size_t elem(int dtype) { return dtype == LPS_DTYPE_F32 ? 4 : 2; }
+int fail(const char* entry, int rc) {
+  fprintf(stderr, "run_case: %s returned %d\n", entry, rc);
+  return 3;
+}
+
+// IN: header {0x4C4D4844, dtype, out_dtype, M, V, H}, x [M * H], w [V * H].
+// OUT: out [M * V] (out_dtype), stats f32[M * ceil(V / 128) * 2].
+int run_lm_head(const std::vector<int32_t>& h, FILE* f, const char* path) {
+  const int M = h[3], V = h[4], H = h[5];
+  uint8_t* x = exact(rd<uint8_t>(f, (size_t)M * H * 2));
+  uint8_t* w = exact(rd<uint8_t>(f, (size_t)V * H * 2));
+  const std::vector<uint8_t> out0((size_t)M * V * elem(h[2]), 0x5A);
+  const std::vector<float> stats0((size_t)M * ((V + 127) / 128) * 2, -7.0f);
+  uint8_t* out = exact(out0);
+  float* stats = exact(stats0);
+  lps_lm_head_args a{};
+  a.x = x;
+  a.w = w;
+  a.out = out;
+  a.stats = stats;
+  a.dtype = h[1];
+  a.out_dtype = h[2];
+  a.rows = M;
+  a.vocab = V;
+  a.hidden = H;
+  a.x_stride = a.w_stride = H;
+  a.out_stride = V;
+  const int rc = lps_lm_head(&a, nullptr);
+  if (rc != LPS_OK) return fail("lps_lm_head", rc);
+  FILE* o = fopen(path, "wb");
+  if (!o) return 2;
+  fwrite(out, 1, out0.size(), o);
+  fwrite(stats, sizeof(float), stats0.size(), o);
+  fclose(o);
+  free(x);
+  free(w);
+  free(out);
+  free(stats);
+  return 0;
+}
+
+// IN: header {0x534D4158, dtype, rows, cols, off, stride, causal, row_offset,
+// stats_cols}, x [off + (rows - 1) * stride + cols], stats f32[rows * G * 2] (stats_cols > 0,
+// G = ceil(cols / stats_cols)).  Row 0 starts at element off of x and of out;
+// the bytes of its 16-byte line that lie 8 or more before it are poisoned.
+// OUT: out (x's elements, 0x5A where nothing was written), lse f32[rows].
+int run_softmax(const std::vector<int32_t>& h, FILE* f, const char* path) {
+  const int dtype = h[1], rows = h[2], cols = h[3], off = h[4], stride = h[5], sc = h[8];
+  const size_t es = elem(dtype), n = off + (size_t)(rows - 1) * stride + cols;
+  const size_t G = sc > 0 ? (cols + sc - 1) / sc : 0;
+  uint8_t* x = exact(rd<uint8_t>(f, n * es));
+  float* stats = exact(rd<float>(f, rows * G * 2));
+  const std::vector<uint8_t> out0(n * es, 0x5A);
+  uint8_t* out = exact(out0);
+  const std::vector<float> lse0(rows, -7.0f);
+  float* lse = exact(lse0);
+  const size_t lead = (size_t)off * es / 8 * 8;
+  __asan_poison_memory_region(x, lead);
+  __asan_poison_memory_region(out, lead);
+  lps_softmax_args a{};
+  a.x = x + (size_t)off * es;
+  a.out = out + (size_t)off * es;
+  a.dtype = dtype;
+  a.rows = rows;
+  a.cols = cols;
+  a.x_stride = a.out_stride = stride;
+  a.causal = h[6];
+  a.seq_len = rows;
+  a.row_offset = h[7];
+  a.row_lse = lse;
+  a.workspace_bytes = lps_softmax_workspace_bytes(rows, cols, dtype);
+  void* ws = a.workspace_bytes ? calloc(1, a.workspace_bytes) : nullptr;
+  a.workspace = ws;
+  if (sc > 0) {
+    a.row_stats = stats;
+    a.stats_stride = (int64_t)G * 2;
+    a.stats_cols = sc;
+  }
+  const int rc = lps_softmax(&a, nullptr);
+  if (rc != LPS_OK) return fail("lps_softmax", rc);
+  __asan_unpoison_memory_region(x, lead);
+  __asan_unpoison_memory_region(out, lead);
+  FILE* o = fopen(path, "wb");
+  if (!o) return 2;
+  fwrite(out, 1, n * es, o);
+  fwrite(lse, sizeof(float), rows, o);
+  fclose(o);
+  free(x);
+  free(stats);
+  free(out);
+  free(lse);
+  free(ws);
+  return 0;
+}
+
+// IN: header {0x53504543, dtype, B, k, V, residual}, f32 {temperature, top_p},
+// target [B * (k + 1) * V], draft [B * k * V], draft tokens i64[B * k],
+// u_accept f32[B * k], u_resample f32[B * (k + 1)].
+// OUT: n_accepted i32[B], tokens i64[B * (k + 1)], status i32[B * (2 k + 1)].
+int run_spec(const std::vector<int32_t>& h, FILE* f, const char* path) {
+  const int dtype = h[1], B = h[2], k = h[3], V = h[4];
+  const size_t es = elem(dtype), Rt = (size_t)B * (k + 1), Rd = (size_t)B * k;
+  const auto tp = rd<float>(f, 2);
+  uint8_t* t = exact(rd<uint8_t>(f, Rt * V * es));
+  uint8_t* d = exact(rd<uint8_t>(f, Rd * V * es));
+  const auto tok = rd<int64_t>(f, Rd);
+  const auto ua = rd<float>(f, Rd), ur = rd<float>(f, Rt);
+  std::vector<int32_t> n_acc(B, -7), status(Rt + Rd, -7);
+  std::vector<int64_t> tokens(Rt, -7);
+  lps_spec_args a{};
+  a.target_logits = t;
+  a.target_stride_b = (int64_t)(k + 1) * V;
+  a.target_stride_k = V;
+  a.draft_logits = d;
+  a.draft_stride_b = (int64_t)k * V;
+  a.draft_stride_k = V;
+  a.dtype = dtype;
+  a.batch = B;
+  a.k = k;
+  a.vocab = V;
+  a.temperature = tp[0];
+  a.top_p = tp[1];
+  a.residual = h[5];
+  a.draft_tokens = tok.data();
+  a.u_accept = ua.data();
+  a.u_resample = ur.data();
+  a.n_accepted = n_acc.data();
+  a.tokens = tokens.data();
+  a.row_status = status.data();
+  a.workspace_bytes = lps_spec_workspace_bytes(B, k, V);
+  void* ws = calloc(1, a.workspace_bytes);
+  a.workspace = ws;
+  const int rc = lps_spec_verify(&a, nullptr);
+  if (rc != LPS_OK) return fail("lps_spec_verify", rc);
+  FILE* o = fopen(path, "wb");
+  if (!o) return 2;
+  wr(o, n_acc);
+  wr(o, tokens);
+  wr(o, status);
+  fclose(o);
+  free(t);
+  free(d);
+  free(ws);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -50,6 +207,9 @@ int main(int argc, char** argv) {
   FILE* f = fopen(argv[1], "rb");
   if (!f) return 2;
   const std::vector<int32_t> h = rd<int32_t>(f, 16);
+  if (h[0] == 0x4C4D4844) return run_lm_head(h, f, argv[2]);
+  if (h[0] == 0x534D4158) return run_softmax(h, f, argv[2]);
+  if (h[0] == 0x53504543) return run_spec(h, f, argv[2]);
   if (h[0] != 0x4C505345) return 2;
   const int dtype = h[1], R = h[2], V = h[3], H = h[4], n_top = h[5], flags = h[6], use_ws = h[7], lp = h[8];
   const int want_h = h[9], skip_draw = h[10];

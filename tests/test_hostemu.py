@@ -70,6 +70,35 @@ def run_case():
     return exe
 
 
+def _exec(exe, inp, out):
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=1",
+               UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
+    r = subprocess.run([exe, str(inp), str(out)], capture_output=True, text=True, timeout=600, env=env)
+    assert r.returncode == 0, f"host run failed ({r.returncode}):\n{r.stderr[-6000:]}"
+    return open(out, "rb").read()
+
+
+def _call(exe, tmp_path, header, *arrays):
+    """One call of another entry point: its output bytes."""
+    inp, out = tmp_path / "in.bin", tmp_path / "out.bin"
+    with open(inp, "wb") as f:
+        f.write(struct.pack("<16i", *header, *[0] * (16 - len(header))))
+        for t in arrays:
+            f.write((t.view(torch.int16) if t.element_size() == 2 else t).contiguous().numpy().tobytes())
+    return _exec(exe, inp, out)
+
+
+def _split(b, *parts):
+    """Output bytes as tensors: (dtype, count) each."""
+    res, o = [], 0
+    for dtype, n in parts:
+        t = torch.empty((n,), dtype=dtype)
+        res.append(torch.frombuffer(bytearray(b[o:o + n * t.element_size()]), dtype=dtype))
+        o += n * t.element_size()
+    assert o == len(b)
+    return res
+
+
 def _run(exe, w, tmp_path, flags=0, workspace=True, logprobs=False, n_top=0, entropy=False, skip_draw=False):
     """One lps_sample call of workload w under the sanitizers; its outputs as a
     SampleOutput-like namespace of CPU tensors."""
@@ -89,11 +118,7 @@ def _run(exe, w, tmp_path, flags=0, workspace=True, logprobs=False, n_top=0, ent
             f.write(w.histories.numpy().astype(np.int32).tobytes())
             f.write(w.hist_len.numpy().astype(np.int32).tobytes())
         f.write(w.uniforms.numpy().astype(np.float32).tobytes())
-    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=1",
-               UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
-    r = subprocess.run([exe, str(inp), str(out)], capture_output=True, text=True, timeout=600, env=env)
-    assert r.returncode == 0, f"host run failed ({r.returncode}):\n{r.stderr[-6000:]}"
-    b = open(out, "rb").read()
+    b = _exec(exe, inp, out)
     o = 0
 
     def take(dt, n):
@@ -402,3 +427,102 @@ def test_history_ids_past_an_odd_vocabulary(run_case, tmp_path, dtype, V):
     assert (got.row_path == 0).all() and (want.row_path == 0).all(), (got.reasons, want.reasons)
     assert torch.equal(got.tokens, want.tokens) and torch.equal(got.status, want.status)
     assert torch.equal(got.kept_count, want.kept_count) and torch.equal(got.kept_cut, want.kept_cut)
+
+
+@pytest.mark.parametrize("M", [1, 33, 65, 97, 129, 257])
+@pytest.mark.parametrize("V,H,dtype,out_dtype", [(301, 80, torch.bfloat16, torch.bfloat16),   # a stage and a part of one
+                                                 (260, 48, torch.float16, torch.float32)])    # less than a stage
+def test_lm_head_tiles(run_case, tmp_path, M, V, H, dtype, out_dtype):
+    """The LM head's LDS ring, its chunk permutation, the columns past the last
+    whole stage, clamped rows and the epilogue's edges, once per tile shape: in
+    bounds; logits within one rounding of the output type and the fp32
+    accumulation (1e-6 sqrt(H)), the block maxima exact and the sums within 2e-6."""
+    g = torch.Generator().manual_seed(M + V + H)
+    x = torch.randn((M, H), generator=g).to(dtype)
+    w = (torch.randn((V, H), generator=g) * (2.0 / H ** 0.5)).to(dtype)
+    G = (V + 127) // 128
+    out, st = _split(_call(run_case, tmp_path, (0x4C4D4844, DT[dtype], DT[out_dtype], M, V, H), x, w),
+                     (out_dtype, M * V), (torch.float32, M * G * 2))
+    out, st = out.reshape(M, V).double(), st.reshape(M, G, 2).double()
+    ref = x.double() @ w.double().T
+    ulp = {torch.bfloat16: 2 ** -8, torch.float32: 2 ** -23}[out_dtype]
+    assert bool(((out - ref).abs() <= ulp * ref.abs() + 1e-6 * H ** 0.5).all())
+    blocks = torch.cat([out, torch.full((M, G * 128 - V), float("-inf"), dtype=torch.float64)], 1).reshape(M, G, 128)
+    mx = blocks.max(dim=2).values
+    assert torch.equal(st[..., 0], mx)
+    torch.testing.assert_close(st[..., 1], torch.exp(blocks - mx.unsqueeze(-1)).sum(dim=2), rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("dtype,rows,cols,off,stride,causal,stats", [
+    (torch.float32, 5, 263, 3, 271, False, False),      # wave kernel, whole rows
+    (torch.bfloat16, 9, 1601, 5, 1603, True, False),    # wave kernel under a mask, rows at other offsets
+    (torch.float32, 257, 1, 3, 1, False, False),        # one element
+    (torch.float16, 3, 129, 5, 131, True, False),       # little work: the three-pass kernel
+    (torch.float16, 3, 5001, 6, 5001, True, False),     # one chunk per row
+    (torch.float32, 2, 4097, 3, 4099, False, False),
+    (torch.bfloat16, 5, 771, 7, 779, False, True),      # from block statistics: 2 and 8 vectors a lane
+    (torch.float32, 2, 4097, 3, 4099, False, True)])
+def test_softmax_misaligned_rows(run_case, tmp_path, dtype, rows, cols, off, stride, causal, stats):
+    """Misaligned rows of the register kernels and of the pass over block
+    statistics: nothing outside a row is read (past the buffer's ends) or
+    written; probabilities within a rounding of the type and 4e-6 (exponents of
+    up to 32 in fp32: 32 * 2^-24 ln 2, three more roundings), log-sum-exp 1e-5."""
+    g = torch.Generator().manual_seed(cols)
+    n = off + (rows - 1) * stride + cols
+    buf = (torch.randn((n,), generator=g) * 3.0).to(dtype)
+    x = torch.as_strided(buf, (rows, cols), (stride, 1), off).double()
+    ro = max(0, cols - rows)
+    G = (cols + 127) // 128 if stats else 0
+    st = torch.zeros((rows, G, 2))
+    if stats:
+        b = torch.cat([x, torch.full((rows, G * 128 - cols), float("-inf"), dtype=torch.float64)], 1).reshape(rows, G, 128)
+        st[..., 0] = b.max(dim=2).values
+        st[..., 1] = torch.exp(b - b.max(dim=2, keepdim=True).values).sum(dim=2)
+    out, lse = _split(_call(run_case, tmp_path, (0x534D4158, DT[dtype], rows, cols, off, stride, int(causal), ro,
+                                                 128 if stats else 0), buf, st),
+                      (dtype, n), (torch.float32, rows))
+    if causal:
+        x = x.masked_fill(torch.arange(cols).unsqueeze(0) > torch.arange(rows).unsqueeze(1) + ro, float("-inf"))
+    tol = {torch.float32: 4e-6, torch.bfloat16: 2 ** -8, torch.float16: 2 ** -10}[dtype]
+    torch.testing.assert_close(torch.as_strided(out, (rows, cols), (stride, 1), off).double(), torch.softmax(x, dim=-1),
+                               atol=1e-7, rtol=tol)
+    torch.testing.assert_close(lse.double(), torch.logsumexp(x, dim=-1), atol=1e-5, rtol=1e-6)
+    beside = torch.ones((n,), dtype=torch.bool)
+    torch.as_strided(beside, (rows, cols), (stride, 1), off).fill_(False)
+    assert bool((out.view(torch.uint8).reshape(n, -1)[beside] == 0x5A).all())
+
+
+@pytest.mark.parametrize("dtype,V,top_p", [(torch.bfloat16, 5001, 1.0), (torch.float32, 4100, 0.9)])
+def test_leviathan_residual(run_case, tmp_path, dtype, V, top_p):
+    """The residual kernels on rows of two chunks (odd and whole vectors; the
+    cut inside ties), in bounds; the drawn id's interval of the cumulative
+    residual in fp64 holds u times the total up to 2e-6 of it."""
+    from oracle import reference_semantics as O
+    B, k, T = 2, 1, 0.8
+    sw = W.c4(B=B, k=k, V=V, seed=V, temperature=T, top_p=top_p)
+    t, d = ((x / 0.25).round().mul(0.25).to(dtype) for x in (sw.target, sw.draft))
+    tok = d.float().argmax(-1)
+    ua = (0.9 + 0.0999 * sw.u_accept).float()
+    n, tokens, status = _split(
+        _call(run_case, tmp_path, (0x53504543, DT[dtype], B, k, V, 1), torch.tensor([T, top_p]), t, d, tok.long(), ua,
+              sw.u_resample.float()), (torch.int32, B), (torch.int64, B * (k + 1)), (torch.int32, B * (2 * k + 1)))
+    assert bool((status == 0).all())
+
+    def kept(x):
+        z = (x.float() / T).double().numpy()
+        order, _, m = O.top_p_truth(torch.from_numpy(z), top_p) if top_p < 1 else (np.arange(V), None, V)
+        e = np.zeros(V)
+        e[order[:m]] = np.exp(z[order[:m]] - z.max())
+        return e / e.sum()
+
+    drawn = 0
+    for b in range(B):
+        j = int(n[b])
+        if j == k:
+            continue
+        r = np.maximum(kept(t[b, j]) - kept(d[b, j]), 0.0)
+        cum = np.cumsum(r)
+        got, u = int(tokens.reshape(B, k + 1)[b, j]), float(sw.u_resample[b, j]) * cum[-1]
+        assert r[got] > 0 and cum[got] - r[got] - 2e-6 * cum[-1] <= u <= cum[got] + 2e-6 * cum[-1], (b, j, got)
+        drawn += 1
+    assert drawn > 0
