@@ -654,12 +654,17 @@ __device__ __forceinline__ double typical_dmin(double Z, double AH, float R, flo
 
 // ---------------------------------------------------------------------------
 // The chunk: NE logits per thread, as NV vectors of VPE logits: slot s = i * VPE
-// + e of thread t is logit (v0 + t + i * NT) * VPE + e of the row.  MA: rows
-// that are not whole aligned vectors (an odd vocabulary starts every row
-// elsewhere in its 16-byte line).  Vectors then count from the line that holds
-// the row's first logit, `mis` logits into it; slots before and after the row
-// are -inf.  A build of its own: with both in one, by a uniform branch or with
-// the clamps always on, aligned batches lost 2 % (c2 38.5 -> 39.3 us).
+// + e of a thread is logit (v0 + t + i * NT) * VPE + e of the row, t = first(),
+// the thread's id.  MA: rows that are not whole aligned vectors (an odd
+// vocabulary starts every row elsewhere in its 16-byte line).  Vectors then
+// count from the line that holds the row's first logit, `mis` logits into it;
+// slots before and after the row are -inf.  A build of its own: with both in
+// one, by a uniform branch or with the clamps always on, aligned batches lost
+// 2 % (c2 38.5 -> 39.3 us).
+// In short MA chunks (one vector a thread at most) first() counts an even split
+// of the vectors over the waves, so that no wave's list segment fills while
+// others are empty: with the first wave holding the whole row, 48 of 64 rows of
+// 401 bf16, top_k 50, went to the general kernel, 53 us (29 so).
 // ---------------------------------------------------------------------------
 template <int DT, int VPE, int NE, bool MA>
 struct Chk {
@@ -668,13 +673,30 @@ struct Chk {
   static_assert(NE % VPE == 0, "whole vectors");
   static_assert(VPE * ES == 16, "16-byte vectors");
   float x[NE];
+  int t0;  // MA: the thread's first vector in the chunk (NT: it holds none)
+
+  __device__ __forceinline__ int first() const { return MA ? t0 : (int)threadIdx.x; }
+  // The first vector of wave w in a short chunk of nv; wave w + 1's follows w's last.
+  __device__ __forceinline__ static int wave_first(int w, int nv) { return w * nv / NW; }
+  // Vectors of wave w in a chunk of nv (MA).
+  __device__ __forceinline__ static int wave_vectors(int w, int nv) {
+    if (nv <= NT) return wave_first(w + 1, nv) - wave_first(w, nv);
+    return nv / NT * 64 + min(max(nv % NT - 64 * w, 0), 64);
+  }
 
   // Issues every load before any use; vectors past the chunk end read the
   // chunk's last vector (MA: a whole vector of the row) and become -inf.  line:
   // the row's first 16-byte line.  MA: the row's first and last vector, when
   // they hold logits of other rows (or none), are read logit by logit.
   __device__ __forceinline__ void load(const char* line, int v0, int nv, int mis, int V) {
-    const int t = threadIdx.x;
+    if constexpr (MA) {
+      t0 = threadIdx.x;
+      if (nv <= NT) {
+        const int w = (int)threadIdx.x >> 6, f = wave_first(w, nv) + ((int)threadIdx.x & 63);
+        t0 = f < wave_first(w + 1, nv) ? f : NT;
+      }
+    }
+    const int t = first();
     const int end = mis + V;
     const int f0 = mis ? 1 : 0, f1 = end / VPE - 1;   // the row's whole vectors
     const int lo = f0 - v0, hi = min(nv - 1, f1 - v0);
@@ -718,7 +740,7 @@ struct Chk {
   // Vector vec of the row (the chunk's q-th), logit by logit.
   __device__ __forceinline__ void partial(const char* line, int vec, int q, int mis, int end) {
     const int iv = q / NT;   // uniform
-    if ((int)threadIdx.x != q % NT) return;
+    if (first() != q % NT) return;
     float f[VPE];
 #pragma unroll
     for (int e = 0; e < VPE; e++) {
@@ -734,14 +756,14 @@ struct Chk {
   }
   // Vocabulary index of slot s (e0 = v0 * VPE - mis; outside [0, V) only where
   // the slot is -inf padding).
-  __device__ static __forceinline__ int index(int e0, int s) {
-    return e0 + ((int)threadIdx.x + (s / VPE) * NT) * VPE + (s % VPE);
+  __device__ __forceinline__ int index(int e0, int s) const {
+    return e0 + (first() + (s / VPE) * NT) * VPE + (s % VPE);
   }
   // Illegal ids to -inf from the row's legality bits (nb bytes; one byte holds
   // a vector's bits when the row is aligned, two when it is not).
   __device__ __forceinline__ void mask(const uint8_t* am, int nb, int v0, int nv, int mis) {
     if (!am) return;
-    const int t = threadIdx.x;
+    const int t = first();
     uint32_t b[NV];
     if constexpr (!MA) {
 #pragma unroll
@@ -822,7 +844,7 @@ template <int DT, int VPE, int NE, bool MA>
 __device__ __forceinline__ void apply_counts(Chk<DT, VPE, NE, MA>& C, const uint32_t* hc, int nv, float rep, float pres,
                                              float freq) {
   constexpr int NV = Chk<DT, VPE, NE, MA>::NV;
-  const int t = threadIdx.x;
+  const int t = C.first();
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const int vl = t + i * NT;

@@ -73,14 +73,30 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     for (int i = 0; i < HB * 8 / 16 / NT; i++) h4[i * NT + tid] = u32x4{0u, 0u, 0u, 0u};
   }
   const float M = bred(tm, S.f, OpMax{});
-  // the m-th largest thread maximum of each wave that holds vectors (a short
-  // row fills the first ones only), m = ceil(k / waves): at least k logits of
-  // the chunk reach the least of them
+  // the m-th largest thread maximum of each wave, m = ceil(k / waves): at least k
+  // logits of the chunk reach the least of them.  MA chunks: waves hold different
+  // numbers of vectors, and m is in proportion (the emptiest would set a low
+  // threshold; 16 rows of 3001 fp32, top_k 100: 26.0 us with equal m); in short
+  // ones of the maxima of a vector's halves, since m may pass the lanes in use
   auto kth_bound = [&](int k) -> uint32_t {
-    const int nw = MA ? max(min(NW, (nv + 63) >> 6), 1) : NW;
-    const uint32_t v1[1] = {f2key(tm)};
-    const uint32_t wth = wave_kth_largest<1>(v1, (uint32_t)((k + nw - 1) / nw));
-    return bred(!MA || wv < nw ? wth : 0xFFFFFFFFu, S.u, OpMin{});
+    const int c = MA ? CK::wave_vectors(wv, nv) : 1, n = MA ? max(nv, 1) : NW;
+    const uint32_t m = (uint32_t)((k * c + n - 1) / n);
+    uint32_t wth;
+    if (MA && nv <= NT) {   // uniform
+      uint32_t v2[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        float mh = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < VPE / 2; e++) mh = fmaxf(mh, C.x[h * (VPE / 2) + e]);
+        v2[h] = f2key(mh);
+      }
+      wth = wave_kth_largest<2>(v2, max(m, 1u));
+    } else {
+      const uint32_t v1[1] = {f2key(tm)};
+      wth = wave_kth_largest<1>(v1, m);
+    }
+    return bred(!MA || c > 0 ? wth : 0xFFFFFFFFu, S.u, OpMin{});
   };
   // nucleus and pure rows with top-N logprobs: the chunk's N largest logits,
   // sorted, kept in LDS until the candidates are published (the same
@@ -93,7 +109,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     const float xth = fmaxf(key2f(th), -3.40282347e38f);
     uint32_t n = 0;
 #pragma unroll
-    for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(e0, s));
+    for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], C.index(e0, s));
     seg_done(S.l, 0, n);
     __syncthreads();
     int np[2];
@@ -128,7 +144,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     if (tn) {
 #pragma unroll
       for (int s = 0; s < NE; s++)
-        if (C.x[s] != C.x[s]) best = min(best, CK::index(e0, s));
+        if (C.x[s] != C.x[s]) best = min(best, C.index(e0, s));
     }
     const int bnan = bred(best, S.i1, OpMin{});
     __syncthreads();
@@ -140,7 +156,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       if (tm == M) {
 #pragma unroll
         for (int s = 0; s < NE; s++)
-          if (C.x[s] == M) best = min(best, CK::index(e0, s));
+          if (C.x[s] == M) best = min(best, C.index(e0, s));
       }
       // (MA, all -inf: the first id, also where padding precedes it)
       sm.amax = bred(best, S.i2, OpMin{});
@@ -172,7 +188,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       const float xth = fmaxf(key2f(th), -3.40282347e38f);
       uint32_t n = 0;
 #pragma unroll
-      for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], CK::index(e0, s));
+      for (int s = 0; s < NE; s++) seg_put(S.l, 0, !(C.x[s] < xth), n, C.x[s], C.index(e0, s));
       seg_done(S.l, 0, n);
       __syncthreads();
       RG_STAMP(13);
@@ -303,7 +319,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
       if (tm >= xlo) {
 #pragma unroll
         for (int s = 0; s < NE; s++)
-          if (C.x[s] >= xlo) best = min(best, CK::index(e0, s));
+          if (C.x[s] >= xlo) best = min(best, C.index(e0, s));
       }
       sm.amax = bred(best, S.i1, OpMin{});
     }
@@ -321,7 +337,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
           nq += inf ? 1u : 0u;
           mq = inf ? mq : fminf(mq, C.x[q * VPE + e]);   // (used for rows without -inf)
         }
-        const bool inr = tid + q * NT < nv;  // (vector q of this thread)
+        const bool inr = C.first() + q * NT < nv;  // (vector q of this thread)
         ni += inr ? nq : 0u;
         mn = inr ? fminf(mn, mq) : mn;
       }
@@ -501,7 +517,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
         float mk = INFINITY;
 #pragma unroll
         for (int s = 0; s < NE; s++) {
-          const bool inr = tid + (s / VPE) * NT < nv;
+          const bool inr = C.first() + (s / VPE) * NT < nv;
           nd += inr && C.x[s] < xt && C.x[s] != -INFINITY ? 1u : 0u;   // (such a row holds no -inf: padding)
           mk = inr && C.x[s] >= xt ? fminf(mk, C.x[s]) : mk;
         }
@@ -854,8 +870,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const int s2 = 2 * k + h;
-          seg_put(S.l, 0, o[h][0], n1, C.x[s2], CK::index(e0, s2));
-          seg_put(S.l, 1, o[h][1], n2, C.x[s2], CK::index(e0, s2));
+          seg_put(S.l, 0, o[h][0], n1, C.x[s2], C.index(e0, s2));
+          seg_put(S.l, 1, o[h][1], n2, C.x[s2], C.index(e0, s2));
         }
       }
     } else {
@@ -866,8 +882,8 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           const int s2 = 2 * k + h;
-          seg_put(S.l, 0, (t1 >> (16 * h) & 0xFFFFu) != 0u, n1, C.x[s2], CK::index(e0, s2));
-          seg_put(S.l, 1, (t2 >> (16 * h) & 0xFFFFu) != 0u, n2, C.x[s2], CK::index(e0, s2));
+          seg_put(S.l, 0, (t1 >> (16 * h) & 0xFFFFu) != 0u, n1, C.x[s2], C.index(e0, s2));
+          seg_put(S.l, 1, (t2 >> (16 * h) & 0xFFFFu) != 0u, n2, C.x[s2], C.index(e0, s2));
         }
       }
     }
@@ -1750,9 +1766,9 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
 // The kernel: grid of ceil(R / 8) * 8 * G workgroups of NT threads.
 // ===========================================================================
 // XF: the launch asks for the entropy output, may hold pure rows without a
-// draw (the mass-only path), or may hold min-p / typical-p rows without top-k
-// or rows with top_k past FAST_KMAX; that code is absent otherwise (such rows
-// are then deferred).
+// draw (the mass-only path), rows without top-k that want top-N logprobs,
+// min-p / typical-p rows without top-k or rows with top_k past FAST_KMAX; that
+// code is absent otherwise (such rows are then deferred).
 template <int DT, int VPE, int NE, bool XF, bool MA>
 __global__ __launch_bounds__(NT) void rowgroup_kernel(RgParams F) {
   __shared__ RgShared<NE> SU;

@@ -429,6 +429,22 @@ def test_history_ids_past_an_odd_vocabulary(run_case, tmp_path, dtype, V):
     assert torch.equal(got.kept_count, want.kept_count) and torch.equal(got.kept_cut, want.kept_cut)
 
 
+@pytest.mark.parametrize("V,dtype", [(129, torch.bfloat16), (401, torch.float32), (1025, torch.float16), (1601, torch.bfloat16)])
+def test_short_misaligned_rows(run_case, tmp_path, V, dtype):
+    """Rows of one vector a thread or less, off the 16-byte lines: their vectors
+    are spread over the waves, so that top_k up to 200 and nucleus rows fit
+    the waves' lists and finish on the row-group kernel."""
+    B = 12
+    w = _small(V, B, dtype, seed=V)
+    i = torch.arange(B)
+    w.top_k = torch.tensor([1, 7, 50, 64, 100, 128, 160, 200, 0, 0, 0, 0], dtype=torch.int32).clamp(max=V - 1)
+    w.top_p = torch.where(i < 8, torch.tensor(1.0), torch.tensor([0.5, 0.9, 0.95, 0.99])[i % 4])
+    w.temperature, w.min_p, w.typical_p = torch.full((B,), 0.9), torch.zeros(B), torch.ones(B)
+    out = _run(run_case, w, tmp_path)
+    assert (out.row_path == 0).all(), out.reasons
+    PY.check_rows(w, out)
+
+
 @pytest.mark.parametrize("M", [1, 33, 65, 97, 129, 257])
 @pytest.mark.parametrize("V,H,dtype,out_dtype", [(301, 80, torch.bfloat16, torch.bfloat16),   # a stage and a part of one
                                                  (260, 48, torch.float16, torch.float32)])    # less than a stage
