@@ -126,8 +126,18 @@ RgPlan rg_plan(int dtype, bool vec, int R, int V, bool lean = false) {
     const int wide = p.vpe == 4 ? 100 : 104;
     if (chunks(wide) < chunks(80) && (long)((R + 7) / 8 * 8) * chunks(80) > (long)device_cus()) p.ne = wide;
   }
+  // misaligned rows: the fewest logits per thread that take no more resident
+  // rounds than 80 would (64 nucleus rows of 20001 bf16: 32.7 us at 80, 28.2 at
+  // 40; of 151643, one round against two: 42.0, 69.2), 24 where that takes no
+  // chunk more than 40 (of 5001: 24.7, 25.8).  Small batches keep 24 while half
+  // the CUs hold their chunks (13 rows of 151643 fp32: 33.9 at 24, 32.2 at 40)
+  const long rows = (R + 7) / 8 * 8, cus = device_cus();
+  if (!vec && (p.ne > 24 || rows * chunks(24) > cus / 2)) {
+    auto rounds = [&](int ne) { return (rows * chunks(ne) + cus - 1) / cus; };
+    p.ne = rounds(40) > rounds(80) ? 80 : chunks(24) == chunks(40) ? 24 : 40;
+  }
   // (a misaligned row may need one chunk more than the workspace is sized for)
-  if (!vec && p.ne < 80 && chunks(p.ne) > rg_max_chunks(R, V)) p.ne = 80;
+  if (!vec && p.ne < 80 && chunks(p.ne) > rg_max_chunks(R, V)) p.ne = chunks(40) <= rg_max_chunks(R, V) ? 40 : 80;
   p.G = chunks(p.ne);
   p.ok = p.G >= 1 && p.G <= (vec ? rg::MAXG : rg_max_chunks(R, V)) && V >= 1;
   p.cv = p.ok ? (p.nvec + p.G - 1) / p.G : 1;
@@ -136,9 +146,9 @@ RgPlan rg_plan(int dtype, bool vec, int R, int V, bool lean = false) {
 }
 // The most chunks any dtype's plan uses for (R, V): sizes the workspace.
 int rg_max_chunks(int R, int V) {
-  // (at least one chunk per 512 x 40 logits, while the row fits MAXG of those:
-  // misaligned rows of large batches then fit with room to spare)
-  const int n40 = (V + rg::NT * 40 - 1) / (rg::NT * 40);
+  // (at least what misaligned rows take at 40 logits per thread, while the row
+  // fits MAXG chunks of those)
+  const int n40 = (V + 2 * 7 + rg::NT * 40 - 1) / (rg::NT * 40);
   int g = n40 <= rg::MAXG ? n40 : 1;
   for (const int dtype : {LPS_DTYPE_F32, LPS_DTYPE_BF16}) {
     const RgPlan p = rg_plan(dtype, true, R, V);

@@ -7,7 +7,7 @@
 //
 // IN holds one call's inputs, OUT receives its outputs (layouts below,
 // little-endian); the first word says which entry point: lps_sample,
-// lps_lm_head, lps_softmax or lps_spec_verify.  The workspace is calloc'd at its exact size, so an
+// lps_lm_head, lps_softmax, lps_spec_verify or the host's planning rules.  The workspace is calloc'd at its exact size, so an
 // access past it, past any input or output array, or past an LDS array of a
 // kernel, stops the run with the sanitizer's report.
 #include "../../llm-pipeline_amd/csrc/lps.hip"
@@ -197,6 +197,23 @@ int run_spec(const std::vector<int32_t>& h, FILE* f, const char* path) {
   return 0;
 }
 
+// IN: header {0x504C414E, n}, n queries i32[4]: {0, dtype, R, V} (a row-group
+// plan for misaligned rows).
+// OUT: i32[4] each: {logits per thread, chunks, the workspace's chunks, planned}.
+int run_plan(const std::vector<int32_t>& h, FILE* f, const char* path) {
+  std::vector<int32_t> out;
+  for (int i = 0; i < h[1]; i++) {
+    const auto q = rd<int32_t>(f, 4);
+    const RgPlan p = rg_plan(q[1], false, q[2], q[3]);
+    out.insert(out.end(), {p.ne, p.G, rg_max_chunks(q[2], q[3]), p.ok ? 1 : 0});
+  }
+  FILE* o = fopen(path, "wb");
+  if (!o) return 2;
+  wr(o, out);
+  fclose(o);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -210,6 +227,7 @@ int main(int argc, char** argv) {
   if (h[0] == 0x4C4D4844) return run_lm_head(h, f, argv[2]);
   if (h[0] == 0x534D4158) return run_softmax(h, f, argv[2]);
   if (h[0] == 0x53504543) return run_spec(h, f, argv[2]);
+  if (h[0] == 0x504C414E) return run_plan(h, f, argv[2]);
   if (h[0] != 0x4C505345) return 2;
   const int dtype = h[1], R = h[2], V = h[3], H = h[4], n_top = h[5], flags = h[6], use_ws = h[7], lp = h[8];
   const int want_h = h[9], skip_draw = h[10];

@@ -542,3 +542,34 @@ def test_leviathan_residual(run_case, tmp_path, dtype, V, top_p):
         assert r[got] > 0 and cum[got] - r[got] - 2e-6 * cum[-1] <= u <= cum[got] + 2e-6 * cum[-1], (b, j, got)
         drawn += 1
     assert drawn > 0
+
+
+def _plans(exe, tmp_path, queries):
+    q = torch.tensor(queries, dtype=torch.int32)
+    return _split(_call(exe, tmp_path, (0x504C414E, len(queries)), q), (torch.int32, 4 * len(queries)))[0].reshape(-1, 4)
+
+
+def test_plans_of_misaligned_rows(run_case, tmp_path):
+    """Logits per thread of misaligned batches: the fewest whose workgroups take no
+    more resident rounds (of 256) than 80 per thread would, 24 only where it
+    takes no more chunks than 40 or the batch is small; the chunks fit the
+    workspace at every size, those just past a chunk's logits among them."""
+    edges = [c * 512 * ne + d for c in (1, 2, 3, 7, 8, 15, 16) for ne in (24, 40, 80) for d in (-9, -3, -1, 1, 7, 13)]
+    sizes = sorted({1, 7, 129, 5001, 20001, 32001, 50257, 65025, 100277, 128257, 151643, *edges})
+    batches = [1, 8, 12, 13, 16, 17, 32, 33, 64, 100, 128, 256, 512, 1024]
+    queries = [(0, dt, R, V) for dt in (0, 1, 2) for R in batches for V in sizes]
+    p = _plans(run_case, tmp_path, queries)
+    for (_, dt, R, V), (ne, G, most, ok) in zip(queries, p.tolist()):
+        vpe = 4 if dt == 0 else 8
+        chunks = lambda n: -(-((V + 2 * (vpe - 1)) // vpe) // (512 * (n // vpe)))
+        rounds = lambda n: -(-((R + 7) // 8 * 8 * chunks(n)) // 256)
+        if not ok:                   # (the general kernel takes these)
+            assert V > 16 * 512 * 40 - 14
+            continue
+        assert G == chunks(ne) <= most <= 16, (dt, R, V)
+        small = R <= (16 if dt == 0 else 12) and chunks(24) <= 16 and (R + 7) // 8 * 8 * chunks(24) <= 128
+        want = 80 if rounds(40) > rounds(80) else 24 if chunks(24) == chunks(40) else 40
+        want = 24 if small else want
+        if chunks(want) > most:      # a row that needs a chunk more than the workspace holds
+            want = 40 if chunks(40) <= most else 80
+        assert ne == want, (dt, R, V, ne)
