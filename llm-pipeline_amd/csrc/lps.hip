@@ -453,20 +453,35 @@ hipError_t launch_lmhead(LmHeadParams P, hipStream_t s) {
   hipLaunchKernelGGL((lmhead_kernel<DT, ODT, T, NTL>), dim3((unsigned)(P.tiles + 7) / 8 * 8), dim3(T::NT), 0, s, P);
   return hipGetLastError();
 }
-// The tile shape by row count (figures in lps_lmhead.h): one row tile as long
-// as the weight's pass over HBM is the bound, so that it is read once and
-// streamed past the caches; 129 to 256 rows fill one 256-row tile (160 rows:
-// 363 us, two 128-row tiles 399); up to 384 rows three 128-row tiles beat two
-// of 256 (554 against 619 us), at 512 and 640 rows they do not (759 against
-// 627, 918 against 883).
+// The tile shape by rows and tiles (figures in lps_lmhead.h).  A tile's time
+// grows with its area (H 4096: 22, 28, 37, 40, 63 and 97 us in this order), so a
+// grid whose tiles all run at once takes the smallest shape of which that is
+// true (256 rows of V 8192: 99 us on 32 tiles of 256 x 256, 44 on 128 of 128 x
+// 128).  Larger grids take the shape by their rows: one row tile as long as the
+// weight's pass over HBM is the bound, so that it is read once and streamed past
+// the caches; 129 to 256 rows fill one 256-row tile (160 rows: 363 us, two
+// 128-row tiles 399); up to 384 rows three 128-row tiles beat two of 256 (554
+// against 619 us), at 512 and 640 rows they do not (759 against 627, 918
+// against 883; V 151936).
+constexpr int LMH_SHAPES[6][2] = {{32, 128}, {64, 128}, {96, 128}, {128, 128}, {128, 256}, {256, 256}};
+int lmhead_shape(int M, int V, int cus) {
+  const int by_rows = M <= 32 ? 0 : M <= 64 ? 1 : M <= 96 ? 2 : M <= 128 ? 3 : M > 256 && M <= 384 ? 4 : 5;
+  for (int i = 0; i <= (M > 256 ? 5 : by_rows); i++) {
+    const int bm = LMH_SHAPES[i][0], bn = LMH_SHAPES[i][1];
+    if ((int64_t)((M + bm - 1) / bm) * ((V + bn - 1) / bn) <= cus) return i;
+  }
+  return by_rows;
+}
 template <int DT, int ODT>
 hipError_t launch_lmhead_rows(const LmHeadParams& P, hipStream_t s) {
-  if (P.M <= 32) return launch_lmhead<DT, ODT, LmTile<32, 128, 1, 4, 128, 3, 1>, true>(P, s);
-  if (P.M <= 64) return launch_lmhead<DT, ODT, LmTile<64, 128, 1, 4, 128, 3, 1>, true>(P, s);
-  if (P.M <= 96) return launch_lmhead<DT, ODT, LmTile<96, 128, 1, 4, 64, 5, 1>, true>(P, s);
-  if (P.M <= 128) return launch_lmhead<DT, ODT, LmTile<128, 128, 4, 2, 64, 4, 2>, true>(P, s);
-  if (P.M > 256 && P.M <= 384) return launch_lmhead<DT, ODT, LmTile<128, 256, 2, 2, 64, 2, 1>, false>(P, s);
-  return launch_lmhead<DT, ODT, LmTile<256, 256, 4, 2, 64, 2, 2>, false>(P, s);
+  switch (lmhead_shape(P.M, P.V, device_cus())) {
+    case 0: return launch_lmhead<DT, ODT, LmTile<32, 128, 1, 4, 128, 3, 1>, true>(P, s);
+    case 1: return launch_lmhead<DT, ODT, LmTile<64, 128, 1, 4, 128, 3, 1>, true>(P, s);
+    case 2: return launch_lmhead<DT, ODT, LmTile<96, 128, 1, 4, 64, 5, 1>, true>(P, s);
+    case 3: return launch_lmhead<DT, ODT, LmTile<128, 128, 4, 2, 64, 4, 2>, true>(P, s);
+    case 4: return launch_lmhead<DT, ODT, LmTile<128, 256, 2, 2, 64, 2, 1>, false>(P, s);
+    default: return launch_lmhead<DT, ODT, LmTile<256, 256, 4, 2, 64, 2, 2>, false>(P, s);
+  }
 }
 template <int DT>
 hipError_t dispatch_lmhead(const LmHeadParams& P, int out_dtype, hipStream_t s) {

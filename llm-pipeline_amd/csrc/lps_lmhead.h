@@ -13,8 +13,9 @@
 //
 // What bounds it: up to ~100 rows the weight's one pass over HBM, past ~250
 // rows the matrix cores.  Both want the same thing, loads in flight that cost
-// no registers and no waiting, so one kernel serves both and the tile shape is
-// chosen by the row count (lps_lm_head):
+// no registers and no waiting, so one kernel serves both.  A grid whose tiles
+// all run at once takes the smallest tile of which that is true, others go by
+// their rows (lmhead_shape):
 //   rows <= 32    32 x 128, 4 waves, 3 stages of 128 columns (120 KB)
 //   rows <= 64    64 x 128, 4 waves, 3 stages of 128 columns (144 KB)
 //   rows <= 96    96 x 128, 4 waves, 5 stages of  64 columns (140 KB)
@@ -31,6 +32,9 @@
 // rows, in one process: 4 stages of 32 columns 2697 against 2451, 4 waves of
 // 128 x 128 2521, 128 x 256 with two workgroups per CU 2942, without the
 // priority hint 2531.
+// Small grids (rows x 4096 -> V, us, by the rows' shape and as chosen; 64 x 128
+// tiles through registers): 256 x 1000 99, 24 (46); 256 x 8192 99, 44 (50); 512 x
+// 8192 100, 46 (95); 1024 x 8192 102, 73 (183); 256 x 32000 104, 77 (208).
 #pragma once
 
 #include "lps_common.h"

@@ -198,14 +198,20 @@ int run_spec(const std::vector<int32_t>& h, FILE* f, const char* path) {
 }
 
 // IN: header {0x504C414E, n}, n queries i32[4]: {0, dtype, R, V} (a row-group
-// plan for misaligned rows).
-// OUT: i32[4] each: {logits per thread, chunks, the workspace's chunks, planned}.
+// plan for misaligned rows), {1, M, V, 0} (an LM-head tile shape).
+// OUT: i32[4] each: {logits per thread, chunks, the workspace's chunks, planned},
+// {rows, columns of a tile, shape, 0}.
 int run_plan(const std::vector<int32_t>& h, FILE* f, const char* path) {
   std::vector<int32_t> out;
   for (int i = 0; i < h[1]; i++) {
     const auto q = rd<int32_t>(f, 4);
-    const RgPlan p = rg_plan(q[1], false, q[2], q[3]);
-    out.insert(out.end(), {p.ne, p.G, rg_max_chunks(q[2], q[3]), p.ok ? 1 : 0});
+    if (q[0] == 0) {
+      const RgPlan p = rg_plan(q[1], false, q[2], q[3]);
+      out.insert(out.end(), {p.ne, p.G, rg_max_chunks(q[2], q[3]), p.ok ? 1 : 0});
+    } else {
+      const int s = lmhead_shape(q[1], q[2], device_cus());
+      out.insert(out.end(), {LMH_SHAPES[s][0], LMH_SHAPES[s][1], s, 0});
+    }
   }
   FILE* o = fopen(path, "wb");
   if (!o) return 2;

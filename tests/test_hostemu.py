@@ -573,3 +573,16 @@ def test_plans_of_misaligned_rows(run_case, tmp_path):
         if chunks(want) > most:      # a row that needs a chunk more than the workspace holds
             want = 40 if chunks(40) <= most else 80
         assert ne == want, (dt, R, V, ne)
+
+
+def test_lm_head_tile_rule(run_case, tmp_path):
+    """A grid whose tiles all run at once on 256 CUs has the smallest tile of
+    which that is true; others go by their rows."""
+    queries = [(1, M, V, 0) for M in (1, 32, 33, 64, 96, 97, 128, 129, 256, 257, 384, 385, 512, 1024, 2048, 65535 * 64)
+               for V in (1, 300, 1000, 8192, 16384, 32000, 50257, 151936)]
+    shapes = [(32, 128), (64, 128), (96, 128), (128, 128), (128, 256), (256, 256)]
+    for (_, M, V, _), (bm, bn, i, _) in zip(queries, _plans(run_case, tmp_path, queries).tolist()):
+        tiles = [-(-M // a) * -(-V // b) for a, b in shapes]
+        rows = 0 if M <= 32 else 1 if M <= 64 else 2 if M <= 96 else 3 if M <= 128 else 4 if 256 < M <= 384 else 5
+        fit = [j for j in range(6 if M > 256 else rows + 1) if tiles[j] <= 256]
+        assert (bm, bn) == shapes[i] and i == (fit[0] if fit else rows), (M, V, i)
