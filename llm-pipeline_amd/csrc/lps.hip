@@ -907,21 +907,27 @@ int lps_softmax(const lps_softmax_args* a, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipError_t e;
   // register-resident kernels: every row of x and out starts 16-byte aligned,
-  // or every row of out is misaligned as its row of x is (mis)
+  // or every row of out is misaligned as its row of x is (alike)
   const int vpl = a->dtype == LPS_DTYPE_F32 ? 4 : 8, es = 16 / vpl;
   auto aligned = [&](const void* p, int64_t stride) {
     return reinterpret_cast<uintptr_t>(p) % 16 == 0 && (a->rows <= 1 || stride % vpl == 0);
   };
   const bool al = aligned(a->x, a->x_stride) && aligned(a->out, a->out_stride);
-  const bool mis = !al && reinterpret_cast<uintptr_t>(a->x) % es == 0 &&
-                   (reinterpret_cast<uintptr_t>(a->x) - reinterpret_cast<uintptr_t>(a->out)) % 16 == 0 &&
-                   (a->rows <= 1 || (a->x_stride - a->out_stride) % vpl == 0);
-  const int span = mis ? softmax_span(a->dtype, a->cols) : a->cols;
+  const bool alike = !al && reinterpret_cast<uintptr_t>(a->x) % es == 0 &&
+                     (reinterpret_cast<uintptr_t>(a->x) - reinterpret_cast<uintptr_t>(a->out)) % 16 == 0 &&
+                     (a->rows <= 1 || (a->x_stride - a->out_stride) % vpl == 0);
+  // little work in short 16-bit rows: the masked first and last vector cost more
+  // than the three-pass kernel's extra passes (64 rows of 129 bf16 4.9 us, 3.9
+  // there; 512 of 769 6.0, 5.6; 2048 of 257 5.8, 6.0; fp32 alike or faster)
+  const bool mis = alike && !(vpl == 8 && a->cols <= 1152 && (int64_t)a->rows * a->cols <= 1 << 19);
+  const int span = alike ? softmax_span(a->dtype, a->cols) : a->cols;
   if (a->row_stats) {
     // one streaming pass from the producer's block statistics
     const int nstats = a->stats_cols > 0 ? (int)(((int64_t)a->cols + a->stats_cols - 1) / a->stats_cols) : 0;
     if (a->causal || a->stats_cols < 1 || (a->rows > 1 && a->stats_stride < 2 * (int64_t)nstats)) return LPS_EINVAL;
-    if (al || mis) {
+    // (short misaligned rows are quicker without them: 256 of 257 bf16 5.7 us, 4.3
+    // on the three-pass kernel; 2048 of 513 9.7, 6.6; 256 of 769 5.5, 5.4)
+    if (al || (alike && a->cols > 640 && (a->cols > 1024 || a->rows <= 256))) {
       const int64_t vecs = ((int64_t)span + vpl - 1) / vpl;
       const int nv = vecs > (int64_t)SM_NT * 2 ? 8 : 2;
       S.G = (int)((vecs + (int64_t)SM_NT * nv - 1) / ((int64_t)SM_NT * nv));
@@ -929,9 +935,9 @@ int lps_softmax(const lps_softmax_args* a, void* stream) {
       S.stats_stride = a->rows > 1 ? a->stats_stride : 2 * (int64_t)nstats;
       S.nstats = nstats;
       switch (a->dtype) {
-        case LPS_DTYPE_F32: e = launch_softmax_apply<LPS_DTYPE_F32>(S, nv, mis, s); break;
-        case LPS_DTYPE_BF16: e = launch_softmax_apply<LPS_DTYPE_BF16>(S, nv, mis, s); break;
-        default: e = launch_softmax_apply<LPS_DTYPE_F16>(S, nv, mis, s); break;
+        case LPS_DTYPE_F32: e = launch_softmax_apply<LPS_DTYPE_F32>(S, nv, alike, s); break;
+        case LPS_DTYPE_BF16: e = launch_softmax_apply<LPS_DTYPE_BF16>(S, nv, alike, s); break;
+        default: e = launch_softmax_apply<LPS_DTYPE_F16>(S, nv, alike, s); break;
       }
       return e == hipSuccess ? LPS_OK : LPS_ELAUNCH;
     }

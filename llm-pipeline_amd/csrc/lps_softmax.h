@@ -27,8 +27,9 @@
 //    and a workgroup that times out computes every chunk's record itself
 //    from the row (the same arithmetic, so the same result).
 //  * softmax_kernel: one workgroup per row in three passes (max; sum; output),
-//    for rows whose input and output are misaligned differently, longer rows,
-//    calls without a workspace and in-place calls of split rows.
+//    for rows whose input and output are misaligned differently, little work in
+//    short misaligned 16-bit rows (lps_softmax), longer rows, calls without a
+//    workspace and in-place calls of split rows.
 //
 // Arithmetic of the register kernels, per lane: m = the lane's max, then
 // e = exp2(fma(x, c, -m c)) (c = log2 e) replaces x in the registers, summed in
