@@ -355,6 +355,14 @@ struct SpecWs {
   size_t bytes;
 };
 
+// The residual option's rows without top-p take the general kernel when they are
+// many and short: its two passes over such a row end sooner than the row-group
+// kernel's chain (300 requests x 2 drafts of 32 fp32: 128 us, 195 on the
+// row-group kernel; 8 x 3 of 4096: 51, 60).  A few rows are no faster there (1 x
+// 5 of 4096 bf16: 36, 32), longer ones slower (8 x 3 of 32000: 170, 61).
+constexpr int LEV_GEN_V = 4096;
+constexpr int LEV_GEN_ROWS = 32;
+
 SpecWs spec_layout(void* base, int B, int k, int V) {
   SpecWs w{};
   const size_t Rt = (size_t)B * (k + 1), Rd = (size_t)B * k;
@@ -740,14 +748,15 @@ int lps_spec_verify(const lps_spec_args* a, void* stream) {
     if (!P.row_status) P.row_status = w.status;
   }
   // Both row sets take the fast kernels (rows they cannot finish exactly go to
-  // the general kernel after them).
+  // the general kernel after them), but for the residual option's short rows.
   // Every row shares the temperature and top-p: the row-kind hint that skips
   // the kernel no row needs (T > 0: nucleus or pure rows; else greedy).
-  const int hint = a->temperature > 0.0f ? LPS_FLAG_ROWS_NUCLEUS : LPS_FLAG_ROWS_TOPK;
   const int Rt = B * (k + 1), Rd = B * k;
+  const bool gen = lev && !(a->top_p < 1.0f) && V <= LEV_GEN_V && Rt + Rd > LEV_GEN_ROWS;
+  const int hint = (a->temperature > 0.0f ? LPS_FLAG_ROWS_NUCLEUS : LPS_FLAG_ROWS_TOPK) | (gen ? LPS_FLAG_GENERIC : 0);
   const bool vec = vec_ok(a->target_logits, a->dtype, V, k + 1, a->target_stride_b, a->target_stride_k);
   const bool vec_d = vec_ok(a->draft_logits, a->dtype, V, k, a->draft_stride_b, a->draft_stride_k);
-  if (Rt + Rd <= RG_MAX_ROWS) {
+  if (Rt + Rd <= RG_MAX_ROWS || gen) {
     // both row sets in one launch: the target rows, then the draft rows as
     // the second row segment (their own logits and layout, draws skipped);
     // the outputs of the two sets are contiguous in the workspace

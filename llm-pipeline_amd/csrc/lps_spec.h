@@ -352,8 +352,11 @@ __global__ __launch_bounds__(RES_NT) void residual_draw_kernel(ResParams P) {
   const int f = S.found;
   if (f < 0) return;     // no residual (uniform)
   const double target = S.run;   // inside the chunk
-  res_combine(P, S, row, b, f, G);
-  res_residual<DT, VEC>(P, S, row, f, rr);
+  if (f != c) {          // (uniform; this workgroup holds chunk c's residuals)
+    res_combine(P, S, row, b, f, G);
+    res_residual<DT, VEC>(P, S, row, f, rr);
+  }
+  __syncthreads();       // every thread has read S.found
   if (tid == 0) S.found = -1;
   // the first id whose cumulative residual exceeds the target, in vocabulary
   // order (past rounding: the last with any residual)

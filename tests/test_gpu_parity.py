@@ -614,3 +614,33 @@ def test_leviathan_residual_chunks(dev, dtype, V, top_p, step):
         assert cum[got] - r[got] - 2e-6 * cum[-1] <= u <= cum[got] + 2e-6 * cum[-1], (b, j, got)
         drawn += 1
     assert drawn > 0
+
+
+@pytest.mark.parametrize("dtype,V,top_p", [(torch.float32, 2048, 0.9), (torch.bfloat16, 2051, 0.8),
+                                           (torch.bfloat16, 2051, 1.0), (torch.float32, 8192, 1.0)])
+def test_leviathan_past_one_launch(dev, dtype, V, top_p):
+    """1500 rows (300 requests x 2 drafts: both row sets in several launches),
+    each its own, cuts inside ties, a target and a draft row that cannot be
+    sampled: the same requests verified 20 at a time give the same outputs."""
+    from lps import spec_verify
+    B, k, T = 300, 2, 0.8
+    sw = W.c4(B=B, k=k, V=V, seed=V, temperature=T, top_p=top_p)
+    t, d = ((x / 0.25).round().mul(0.25).to(dtype) for x in (sw.target, sw.draft))
+    t[211, 0, 5] = float("nan")
+    d[299, 0, 7] = float("inf")
+    tok = d.float().nan_to_num(0.0, 0.0).argmax(-1)
+    ua = 0.9 + 0.0999 * sw.u_accept
+
+    def verify(i, j):
+        o = spec_verify(t[i:j].to(dev), d[i:j].to(dev), tok[i:j].to(dev), ua[i:j].to(dev), sw.u_resample[i:j].to(dev),
+                        T, top_p, residual="leviathan")
+        n = (j - i) * (k + 1)     # status: the target rows, then the draft rows
+        s = o.status.reshape(-1)
+        return o.n_accepted, o.tokens, o.accept, s[:n], s[n:]
+
+    whole = verify(0, B)
+    parts = [torch.cat(x) for x in zip(*[verify(i, i + 20) for i in range(0, B, 20)])]
+    for a, b in zip(whole, parts):
+        assert torch.equal(a, b)
+    assert int(whole[3][211 * (k + 1)]) != 0 and int(whole[4][299 * k]) != 0
+    assert int((whole[0] < k).sum()) > B // 4
