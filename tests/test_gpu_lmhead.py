@@ -112,3 +112,22 @@ def test_lm_head_tile_edges(dev, M, V, H, dtype, out_dtype):
     out, stats = lm_head(x.to(dev), w.to(dev), out_dtype=out_dtype, return_stats=True)
     _check_logits(out, _ref(x, w), H, 1.0)
     _check_stats(out, stats)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V", [129, 771, 2055, 4099, 16389, 50257])
+def test_softmax_from_stats_odd_vocabularies(dev, V, out_dtype):
+    """Odd rows (every offset in a 16-byte line) at both vector counts of the
+    pass over the statistics and just past a chunk's end.  Bounds: a rounding of
+    the output type; in fp32 4e-6 (exponents of up to 32: 32 * 2^-24 ln 2, and
+    the roundings of max * log2 e, of the sum and of the product)."""
+    g = torch.Generator().manual_seed(V)
+    M, H = 17, 64
+    x = torch.randn((M, H), generator=g).to(torch.float16).to(dev)
+    w = (torch.randn((V, H), generator=g) * (2.0 / H ** 0.5)).to(torch.float16).to(dev)
+    logits, stats = lm_head(x, w, out_dtype=out_dtype, return_stats=True)
+    p, lse = fused_softmax(logits, row_stats=stats, return_lse=True)
+    exact = logits.double().cpu()
+    tol = {torch.float32: 4e-6, torch.bfloat16: 2 ** -8, torch.float16: 2 ** -10}[out_dtype]
+    torch.testing.assert_close(p.double().cpu(), torch.softmax(exact, dim=-1), atol=1e-7, rtol=tol)
+    torch.testing.assert_close(lse.double().cpu(), torch.logsumexp(exact, dim=-1), atol=2e-5, rtol=1e-6)

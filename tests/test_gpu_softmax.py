@@ -250,8 +250,8 @@ def test_softmax_workspace_reuse_across_layouts(dev):
 @pytest.mark.parametrize("causal", [False, True])
 def test_softmax_rows_off_the_16_byte_lines(dev, dtype, rows, cols, causal):
     """Odd row lengths (every row starts elsewhere in its 16-byte line) at the
-    edges of the wave and chunk plans, whose span counts from that line, and the
-    elements beside the rows left alone; _check's bounds."""
+    edges of the wave and chunk plans, whose span counts from that line, and rows
+    whose input and output are misaligned differently; _check's bounds."""
     g = torch.Generator().manual_seed(rows * cols)
     x = (torch.randn((rows, cols), generator=g) * 4.0).to(dtype)
     off = max(0, cols - rows)
@@ -261,8 +261,41 @@ def test_softmax_rows_off_the_16_byte_lines(dev, dtype, rows, cols, causal):
     if causal:
         xd = xd.masked_fill(torch.arange(cols).unsqueeze(0) > torch.arange(rows).unsqueeze(1) + off, float("-inf"))
     torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(xd, dim=-1), atol=1e-5, rtol=1e-6)
-    big = torch.full((rows * cols + 8,), 7.0, dtype=dtype, device=dev)     # rows from the second element on
+    big = torch.zeros((rows * cols + 8,), dtype=dtype, device=dev)         # rows from the second element on
     big[1:1 + rows * cols] = x.to(dev).reshape(-1)
     out = fused_softmax(big[1:1 + rows * cols].view(rows, cols), causal=causal, row_offset=off)
     _check(out, x, causal=causal, row_offset=off)
-    assert bool((big[:1] == 7).all()) and bool((big[1 + rows * cols:] == 7).all())
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("dtype,rows,cols,off,pad", [(torch.bfloat16, 9, 1601, 7, 9), (torch.float16, 8193, 65, 1, 4),  # a wave a row
+                                                     (torch.float32, 6, 1027, 3, 2),
+                                                     (torch.bfloat16, 5, 8187, 3, 8), (torch.float32, 3, 4099, 1, 1),   # one chunk
+                                                     (torch.bfloat16, 4, 50257, 5, 3), (torch.float32, 3, 20001, 2, 5)])  # split rows
+def test_softmax_misaligned_rows_leave_their_neighbours(dev, dtype, rows, cols, off, pad, in_place):
+    """Rows that start inside a 16-byte line, alike in input and output (the
+    register kernels; in place, split rows take the three-pass kernel): what
+    lies before, between and after the output's rows is left alone."""
+    import ctypes
+    from lps import _device as D, _lib
+    g = torch.Generator().manual_seed(cols)
+    vpl = 16 // torch.empty((), dtype=dtype).element_size()
+    xs = cols + pad
+    os = xs if in_place else xs + 2 * vpl              # (congruent, not equal)
+    x = (torch.randn((rows, cols), generator=g) * 3.0).to(dtype)
+    xb = torch.full((off + rows * xs,), 7.0, dtype=dtype, device=dev)
+    torch.as_strided(xb, (rows, cols), (xs, 1), off).copy_(x)
+    ob = xb if in_place else torch.full((off + rows * os + 3,), 7.0, dtype=dtype, device=dev)
+    before = ob.clone()
+    lse = torch.empty((rows,), device=dev)
+    lib, a = _lib.load(), _lib.SoftmaxArgs()
+    es = 16 // vpl
+    a.x, a.out, a.dtype = xb.data_ptr() + off * es, ob.data_ptr() + off * es, D.dtype_code(xb)
+    a.rows, a.cols, a.x_stride, a.out_stride, a.seq_len, a.row_lse = rows, cols, xs, os, 1, lse.data_ptr()
+    ws = torch.zeros((max(1, lib.lps_softmax_workspace_bytes(rows, cols, a.dtype)),), dtype=torch.uint8, device=dev)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    _lib.check(lib.lps_softmax(ctypes.byref(a), D.stream_of(dev)), "lps_softmax")
+    _check(torch.as_strided(ob, (rows, cols), (os, 1), off), x)
+    torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(x.double(), dim=-1), atol=1e-5, rtol=1e-6)
+    torch.as_strided(before, (rows, cols), (os, 1), off).copy_(torch.as_strided(ob, (rows, cols), (os, 1), off))
+    assert torch.equal(ob, before) and int(ws.count_nonzero()) == 0
