@@ -98,6 +98,10 @@ bool rg_wants_xf(const KParams& k, int flags) {
   return k.entropy || mt || tn || ((k.skip_draw || (k.logits2 && k.skip_draw2)) && (k.top_p != nullptr || !(k.top_p_def < 1.0f)));
 }
 
+// (of this file) the launch's query probabilities to fp32's last bits: the build
+// with the extra features, or the wide plans' own
+constexpr int FLAG_QP = 1 << 30;
+
 // Launch shape of the row-group kernel for a batch: logits per thread (NE) of
 // the instantiated variants, chunks per row (G <= MAXG), vectors per chunk.
 struct RgPlan {
@@ -209,11 +213,13 @@ hipError_t launch_rg(rg::RgParams F, int flags, hipStream_t s) {
   if (run_rg) {
     // the build with the extra features when the launch may need them (the
     // plans of more than 80 logits per thread are made only for the other)
-    if (rg_wants_xf(F.k, flags)) {
+    if (rg_wants_xf(F.k, flags) || (NE <= 80 && (flags & FLAG_QP))) {
       if constexpr (NE <= 80) hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, true, MA>), dim3(grid), dim3(rg::NT), 0, s, F);
       else return hipErrorInvalidValue;
     } else {
-      hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, false, MA>), dim3(grid), dim3(rg::NT), 0, s, F);
+      if (NE > 80 && (flags & FLAG_QP))
+        hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, false, MA, (NE > 80)>), dim3(grid), dim3(rg::NT), 0, s, F);
+      else hipLaunchKernelGGL((rg::rowgroup_kernel<DT, VPE, NE, false, MA, false>), dim3(grid), dim3(rg::NT), 0, s, F);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -753,9 +759,13 @@ int lps_spec_verify(const lps_spec_args* a, void* stream) {
   // the kernel no row needs (T > 0: nucleus or pure rows; else greedy).
   const int Rt = B * (k + 1), Rd = B * k;
   const bool gen = lev && !(a->top_p < 1.0f) && V <= LEV_GEN_V && Rt + Rd > LEV_GEN_ROWS;
-  const int hint = (a->temperature > 0.0f ? LPS_FLAG_ROWS_NUCLEUS : LPS_FLAG_ROWS_TOPK) | (gen ? LPS_FLAG_GENERIC : 0);
+  int hint = (a->temperature > 0.0f ? LPS_FLAG_ROWS_NUCLEUS : LPS_FLAG_ROWS_TOPK) | (gen ? LPS_FLAG_GENERIC : 0);
   const bool vec = vec_ok(a->target_logits, a->dtype, V, k + 1, a->target_stride_b, a->target_stride_k);
   const bool vec_d = vec_ok(a->draft_logits, a->dtype, V, k, a->draft_stride_b, a->draft_stride_k);
+  // (the residual option's probabilities to fp32's last bits, as the general kernel
+  // gave them: query_probability.  After top-p the other build is 4 to 8 % faster
+  // and off by 1.3e-7 of their norm, 3.4e-8 so: 8 x 3 of 151936 bf16 91, 95 us)
+  if (lev) hint |= FLAG_QP;
   if (Rt + Rd <= RG_MAX_ROWS || gen) {
     // both row sets in one launch: the target rows, then the draft rows as
     // the second row segment (their own logits and layout, draws skipped);

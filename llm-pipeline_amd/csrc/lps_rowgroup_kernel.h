@@ -16,9 +16,9 @@ __device__ __forceinline__ bool wait_count(uint32_t* p, uint32_t n) {
 // ===========================================================================
 // Chunk phase.  Returns the row's mode (MODE_DEFER: nothing published).
 // ===========================================================================
-template <int DT, int VPE, int NE, bool XF, bool MA>
+template <int DT, int VPE, int NE, bool XF, bool MA, bool QP>
 __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, const int r, const int j,
-                                           const RowCfg& g, const uint32_t epoch, int& tcase) {
+                                           const RowCfg& g, const uint32_t epoch, int& tcase, float& ybar) {
   using CK = Chk<DT, VPE, NE, MA>;
   const KParams& P = F.k;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -597,6 +597,7 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     {
       int lo = 1 << 30, hi = -1;
       uint32_t nest1 = 0, nest2 = 0;  // elements of the regions (upper estimates: bin mass / the bin's least mass)
+      float qa = 0.0f;                // queried rows: mass times log2 mass, over the bins that hold kept ids
       uint64_t a2 = ~0ull;  // cumulative mass at region 2's top
       double a = sx;
 #pragma unroll
@@ -615,7 +616,12 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
           nest1 += in1 ? n : 0u;
           nest2 += in2 ? n : 0u;
         }
+        if (QP && P.query_prob) qa += !nuc || b >= lo1 ? (float)mrg[i] * bin_log2(b) : 0.0f;
         a += mrg[i];
+      }
+      if (QP && P.query_prob) {
+        qa = wreduce(qa, OpAdd{});
+        if (lane == 0) S.md[4 + wv] = (double)qa;
       }
       if (hi >= 0) {
         atomicMin(&S.mi[2], lo);
@@ -629,6 +635,13 @@ __device__ __forceinline__ int chunk_phase(const RgParams& F, RgChunkS<NE>& S, c
     const int lo2 = S.mi[2];
     const int hi2 = S.mi[3];
     const uint32_t nest1 = S.u3[0], nest2 = S.u3[1];
+    if (QP && P.query_prob) {   // over the mass of those bins
+      double qa = 0.0;
+#pragma unroll
+      for (int i = 0; i < NW; i++) qa += S.md[4 + i];
+      const double qm = nuc ? __builtin_bit_cast(double, q1b) : Z;
+      ybar = qm > 0.0 ? (float)(qa / qm) : 0.0f;
+    }
     if (!(XF && targ) && (hi2 < 0 || !rfin)) flags |= RF_REGION;
     const bool need2 = !row_skips_draw(P, r);
     // ---- crowded regions take the second level (a row-uniform decision: every
@@ -1270,9 +1283,9 @@ __device__ __forceinline__ int topk_decide(const RowCfg& g, int V, const uint64_
   return 0;
 }
 
-template <int DT, int VPE, bool XF>
+template <int DT, int VPE, bool XF, bool QP>
 __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const int r, const RowCfg& g,
-                                           const uint32_t epoch, const int tcase) {
+                                           const uint32_t epoch, const int tcase, const float ybar) {
   const KParams& P = F.k;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int G = F.G;
@@ -1347,7 +1360,8 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
     // (a chunk dl octaves under it: e 2^-dl, log2 e - dl), in log2 units
     // (and typical rows without top-p / min-p, with their -inf count)
     const bool tpl = XF && mode == MODE_NUCLEUS && g.typp < 1.0f && !(g.topp < 1.0f) && !(g.minp > 0.0f) && !g.bigk;
-    const double AH = (XF && (P.entropy || tpl)) ? rreduce16(rfin ? sc * (a.zent - (double)(R - a.ref) * a.zsum) : 0.0, OpAdd{}) : 0.0;
+    // (queried pure rows without a draw: their mean log2 mass)
+    const double AH = (XF && (P.entropy || tpl || (P.query_prob && mode == MODE_PURE))) ? rreduce16(rfin ? sc * (a.zent - (double)(R - a.ref) * a.zsum) : 0.0, OpAdd{}) : 0.0;
     // (a typical cut under the histogram: the dropped logits and the least kept key)
     const bool low = tcase == TYP_LOW;
     const uint32_t ndr = low ? rreduce16(in ? tw_n(a.ab1) : 0u, OpAdd{}) : 0u;
@@ -1675,8 +1689,12 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
       const uint32_t kq = f2key(zq);
       const bool kept = zq != -INFINITY && ((!nuc && tcase != TYP_LOW) || kq > vkey ||
                                             (kq == vkey && (n_tie == kNoTie || qtok <= tie_lim)));
-      // (in the row mass's arithmetic, so that the rounding of c cancels against Z's)
-      if (kept) qprob = XF && targ ? 1.0f : (float)((double)emass(xq, c, Rref) * kFix / (double)Zkept);
+      if constexpr (QP) {
+        const double yb = XF && mode == MODE_PURE && row_skips_draw(P, r) ? S.md[3] / Zfull : (double)ybar;
+        if (kept) qprob = XF && targ ? 1.0f : query_probability(xq, c, T, Rref, yb, (double)Zkept);
+      } else if (kept) {   // in the row mass's arithmetic, so that much of c's rounding cancels against Z's
+        qprob = (float)((double)emass(xq, c, Rref) * kFix / (double)Zkept);
+      }
     }
   }
   if (row_skips_draw(P, r) && !greedy) token = -1;
@@ -1768,8 +1786,9 @@ __device__ __forceinline__ int final_phase(const RgParams& F, RgFinalS& S, const
 // XF: the launch asks for the entropy output, may hold pure rows without a
 // draw (the mass-only path), rows without top-k that want top-N logprobs,
 // min-p / typical-p rows without top-k or rows with top_k past FAST_KMAX; that
-// code is absent otherwise (such rows are then deferred).
-template <int DT, int VPE, int NE, bool XF, bool MA>
+// code is absent otherwise (such rows are then deferred).  QP: query
+// probabilities are corrected for c's rounding (query_probability).
+template <int DT, int VPE, int NE, bool XF, bool MA, bool QP = XF>
 __global__ __launch_bounds__(NT) void rowgroup_kernel(RgParams F) {
   __shared__ RgShared<NE> SU;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -1784,7 +1803,8 @@ __global__ __launch_bounds__(NT) void rowgroup_kernel(RgParams F) {
   // before any of them arrives
   const uint32_t epoch = ld_agent(F.counters + (int64_t)r * 32 + CTR_EPOCH);
   int tcase = -1;  // typical-p rows without other filters: TYP_*
-  const int mode = chunk_phase<DT, VPE, NE, XF, MA>(F, SU.c, r, j, g, epoch, tcase);
+  float ybar = 0.0f;
+  const int mode = chunk_phase<DT, VPE, NE, XF, MA, QP>(F, SU.c, r, j, g, epoch, tcase, ybar);
   if (mode == MODE_DEFER) {
     if (j == 0 && threadIdx.x == 0) F.status[r] = LPS_ROW_DEFERRED | (1 << 8);
     return;
@@ -1802,7 +1822,7 @@ __global__ __launch_bounds__(NT) void rowgroup_kernel(RgParams F) {
   if (!SU.c.mi[7] || threadIdx.x >= FT) return;
   acquire_agent();
   RG_STAMP(24);
-  const int reason = final_phase<DT, VPE, XF>(F, SU.f, r, g, epoch, tcase);
+  const int reason = final_phase<DT, VPE, XF, QP>(F, SU.f, r, g, epoch, tcase, ybar);
   RG_STAMP(31);
   if (reason > 0 && threadIdx.x == 0) F.status[r] = LPS_ROW_DEFERRED | (reason << 8);
 }

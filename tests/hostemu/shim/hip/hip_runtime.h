@@ -324,6 +324,7 @@ template <typename T> inline T atomicCAS(T* p, T cmp, T v) {
 // HW_REG_XCC_ID: the XCD a block id is dispatched to (round-robin over 8)
 #define __builtin_amdgcn_s_getreg(reg) ((int)(::lps_emu::t_block.x & 7u))
 #define __builtin_amdgcn_exp2f(x) exp2f(x)
+#define __builtin_amdgcn_logf(x) log2f(x)
 
 inline uint64_t lps_emu_ballot(bool p) {
   return lps_emu::xchg<uint64_t>(p ? 1ull : 0ull, [](const uint64_t* b, uint64_t alive) {

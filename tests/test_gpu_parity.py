@@ -644,3 +644,38 @@ def test_leviathan_past_one_launch(dev, dtype, V, top_p):
         assert torch.equal(a, b)
     assert int(whole[3][211 * (k + 1)]) != 0 and int(whole[4][299 * k]) != 0
     assert int((whole[0] < k).sum()) > B // 4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,top_p,residual", [(0.8, 1.0, "target"), (0.8, 1.0, "leviathan"), (0.65, 1.0, "leviathan"),
+                                              (1.1, 0.95, "leviathan")])
+def test_spec_verify_probabilities_to_fp32(dev, dtype, T, top_p, residual):
+    """The target's and the draft's probability of every drafted token, against
+    64 bits: 2-norm of the difference within 8e-8 of the values' (fp32 rounds
+    each by up to 6e-8, its masses' sum adds less; log2 e / T in fp32 alone would
+    move them by 0.8e-7, 1.7e-7 and 1.8e-7 at these T)."""
+    from lps import spec_verify
+    B, k, V = 8, 3, 151936
+    g = torch.Generator(device=dev).manual_seed(3)
+    t = torch.randn((B, k + 1, V), generator=g, device=dev) * 2.0
+    d = (t[:, :k] + 0.5 * torch.randn((B, k, V), generator=g, device=dev)).to(dtype)
+    t = t.to(dtype)
+    T32, p32 = float(np.float32(T)), float(np.float32(top_p))
+    tok = torch.multinomial(torch.softmax(d.reshape(B * k, V).float() / T, -1), 1, generator=g).reshape(B, k)
+    u = torch.rand((B, 2 * k + 1), generator=g, device=dev)
+    o = spec_verify(t, d, tok, u[:, :k], u[:, k:], T, top_p, residual=residual)
+
+    def exact(x):
+        z = x.double() / T32
+        v, at = torch.sort(z, dim=-1, descending=True, stable=True)
+        e = (v - v[..., :1]).exp()
+        if top_p < 1.0:
+            c = e.cumsum(-1)
+            e = torch.where(c - e <= p32 * c[..., -1:], e, 0.0)
+        return (e * (at == tok.unsqueeze(-1))).sum(-1) / e.sum(-1)
+
+    for got, x in ((o.p_target, t[:, :k]), (o.q_draft, d)):
+        want = exact(x)
+        err = float((got.double() - want).norm() / want.norm())
+        print(f"{dtype} T {T} top_p {top_p}: {err:.2e}")
+        assert err <= 8e-8
