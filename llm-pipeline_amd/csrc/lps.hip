@@ -150,9 +150,9 @@ RgPlan rg_plan(int dtype, bool vec, int R, int V, bool lean = false) {
 }
 // The most chunks any dtype's plan uses for (R, V): sizes the workspace.
 int rg_max_chunks(int R, int V) {
-  // (at least what misaligned rows take at 40 logits per thread, while the row
-  // fits MAXG chunks of those)
-  const int n40 = (V + 2 * 7 + rg::NT * 40 - 1) / (rg::NT * 40);
+  // (at least one chunk per 512 x 40 logits, while the row fits MAXG of those:
+  // misaligned rows of large batches then fit with room to spare)
+  const int n40 = (V + rg::NT * 40 - 1) / (rg::NT * 40);
   int g = n40 <= rg::MAXG ? n40 : 1;
   for (const int dtype : {LPS_DTYPE_F32, LPS_DTYPE_BF16}) {
     const RgPlan p = rg_plan(dtype, true, R, V);

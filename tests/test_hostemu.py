@@ -553,7 +553,8 @@ def test_plans_of_misaligned_rows(run_case, tmp_path):
     """Logits per thread of misaligned batches: the fewest whose workgroups take no
     more resident rounds (of 256) than 80 per thread would, 24 only where it
     takes no more chunks than 40 or the batch is small; the chunks fit the
-    workspace at every size, those just past a chunk's logits among them."""
+    workspace at every size, those just past a chunk's logits among them, and
+    the workspace holds a chunk per 512 x 40 logits, no more."""
     edges = [c * 512 * ne + d for c in (1, 2, 3, 7, 8, 15, 16) for ne in (24, 40, 80) for d in (-9, -3, -1, 1, 7, 13)]
     sizes = sorted({1, 7, 129, 5001, 20001, 32001, 50257, 65025, 100277, 128257, 151643, *edges})
     batches = [1, 8, 12, 13, 16, 17, 32, 33, 64, 100, 128, 256, 512, 1024]
@@ -567,6 +568,8 @@ def test_plans_of_misaligned_rows(run_case, tmp_path):
             assert V > 16 * 512 * 40 - 14
             continue
         assert G == chunks(ne) <= most <= 16, (dt, R, V)
+        if R > 32 and V <= 16 * 512 * 40:     # (the workspace's size, which no-alloc calls are admitted by)
+            assert most == -(-V // (512 * 40)), (dt, R, V)
         small = R <= (16 if dt == 0 else 12) and chunks(24) <= 16 and (R + 7) // 8 * 8 * chunks(24) <= 128
         want = 80 if rounds(40) > rounds(80) else 24 if chunks(24) == chunks(40) else 40
         want = 24 if small else want
